@@ -64,16 +64,18 @@ HBM_PEAK_GBPS = 8000.0
 LATENCY_SAMPLES = 20
 # MI355X's host link, PCIe 5.0 x16: 32 GT/s x 16 lanes, 128b/130b encoding, per direction.
 PCIE5_X16_GBPS = round(32 * 16 * 128 / 130 / 8, 2)
-# SHA-256 runs one dependency chain per record (two lanes of a round wave).
-# The round wave issues 596 VALU per 64-byte block (counted in the gfx950 ISA
-# of sha256_kernel: 192 alignbit, 192 bitop3, 74 DPP adds, 64 add3, 64 xad,
-# 10 others); a wave64 VALU takes 4 cycles of its SIMD at the 2.4 GHz peak
-# engine clock.  All chains run side by side (one round wave per 32 records).
-# The round's own 9-VALU sequence is also timed live on one wave
-# (kvsnap_sha_round_probe: shader cycles and the 100 MHz constant clock), which
-# gives the rate a slot runs at and the engine clock meanwhile; the bound at
-# that rate is reported beside the nominal one.
-SHA_VALU_PER_BLOCK = 596
+# SHA-256 runs one dependency chain per record (eight lanes of a round wave, the
+# quad form; sessions of more than 1536 records take the two-lane form).  The
+# round wave issues 534 VALU per 64-byte block (the assembly of SHA_BLOCK: 64
+# slots of alignbit, 2 bitop3, xad, 3 DPP, add3, and 22 at the block's turn); a
+# wave64 VALU takes 4 cycles of its SIMD at the 2.4 GHz peak engine clock.  All
+# chains run side by side (one round wave per 8 records).  The two-lane form's
+# 9-VALU slot is also timed live on one wave (kvsnap_sha_round_probe: shader
+# cycles and the 100 MHz constant clock), which gives the rate instructions
+# issue at and the engine clock meanwhile; the bound at that rate (8 of its 9
+# instructions a slot) is reported beside the nominal one.
+SHA_VALU_PER_BLOCK = 534
+SHA_SLOT_VALU, SHA_PROBE_SLOT_VALU = 8, 9
 SHA_CYCLES_PER_VALU = 4
 ENGINE_CLOCK_GHZ = 2.4
 SHA_PROBE_SLOTS = 1 << 18
@@ -117,7 +119,7 @@ def sha_issue_bound(record_bytes, records, ms, round_rate):
     bound_ms = blocks * SHA_VALU_PER_BLOCK * SHA_CYCLES_PER_VALU / (ENGINE_CLOCK_GHZ * 1e6)
     total = record_bytes * records
     slot_cycles, clock_ghz = round_rate
-    sequence_ms = blocks * 64 * slot_cycles / (ENGINE_CLOCK_GHZ * 1e6)
+    sequence_ms = blocks * 64 * slot_cycles * SHA_SLOT_VALU / SHA_PROBE_SLOT_VALU / (ENGINE_CLOCK_GHZ * 1e6)
     fips_ms = blocks * (64 * SHA_FIPS_TWO_LANE_ROUND + SHA_FIPS_FEED_FORWARD) * SHA_CYCLES_PER_VALU / (
         ENGINE_CLOCK_GHZ * 1e6)
     one_lane_ms = blocks * (64 * SHA_FIPS_ROUND_INSTRUCTIONS + 2 * SHA_FIPS_FEED_FORWARD) * SHA_CYCLES_PER_VALU / (
@@ -132,7 +134,8 @@ def sha_issue_bound(record_bytes, records, ms, round_rate):
             "achieved": round(total / (ms * 1e6), 2), "peak": round(total / (bound_ms * 1e6), 2), "unit": "GB/s",
             "frac": round(bound_ms / ms, 4), "round_cycles_measured": round(slot_cycles, 2),
             "round_probe_clock_ghz": round(clock_ghz, 3),
-            "round_probe": "kvsnap_sha_round_probe: the round sequence alone on one wave, s_memtime / s_memrealtime",
+            "round_probe": "kvsnap_sha_round_probe: the two-lane round sequence (9 VALU) alone on one wave, "
+                           "s_memtime / s_memrealtime",
             "round_sequence_bound_ms": round(sequence_ms, 3), "frac_of_round_sequence_rate": round(sequence_ms / ms, 4)}
 
 

@@ -1424,15 +1424,14 @@ __global__ __launch_bounds__(kFinishThreads) void restore_checked_finish_kernel(
 // dozen of the chip's 1024 SIMDs.  A record's time is therefore the time of
 // its chain of rounds (a wave64 VALU instruction takes 4 cycles of its SIMD),
 // and everything that does not depend on the chaining state is moved off it:
-//   * two producer waves (one record per lane, alternate blocks of a step)
-//     load each block a step ahead, byte-swap it, expand the message schedule
-//     and add the round constants (W[t] + K[t]) into LDS;
-//   * two round waves run only the 64 rounds, two lanes per record (the
-//     e-half and the a-half of each round side by side, the a-half one round
-//     behind; see sha_block), 10 VALU per round.
-// Workgroup = two round waves + two producer waves over the same 64 records;
-// the producers fill one half of a double buffer of kShaStep blocks while the
-// round waves read the other.
+//   * producer waves load each block ahead, byte-swap it, expand the message
+//     schedule and add the round constants (W[t] + K[t]) into LDS;
+//   * round waves run only the 64 rounds, the e-half and the a-half of each
+//     round side by side on lanes of their own, the a-half two rounds behind.
+// Two forms share the code (ShaTwoLane and ShaQuad below): two lanes a record
+// and 9 VALU a round, or eight lanes a record and 8 VALU a round.  A workgroup
+// is four waves on one CU; its producers fill one of three buffers of kStep
+// blocks while the round waves read another.
 
 __constant__ uint32_t kSha[64] = {
     0x428a2f98, 0x71374491, 0xb5c0fbcf, 0xe9b5dba5, 0x3956c25b, 0x59f111f1, 0x923f82a4, 0xab1c5ed5,
@@ -1449,7 +1448,6 @@ __device__ __forceinline__ uint32_t rotr(uint32_t x, int n) { return (x >> n) | 
 __device__ __forceinline__ uint32_t bswap(uint32_t x) { return __builtin_bswap32(x); }
 
 constexpr int kShaBlockQuads = 16;  // 64 schedule words per block, read 4 at a time
-constexpr int kShaColumns = 65;     // 64 records, then {1,1,1,1} for the a-lanes
 
 // Block `blk` of a record as 16 big-endian words, FIPS 180-4 padding included:
 // blocks [0, whole) are payload, then 1 or 2 final blocks carry the tail,
@@ -1522,8 +1520,9 @@ __device__ __forceinline__ void sha_message_raw(const uint8_t* __restrict__ p, u
     for (int i = 0; i < 16; ++i) raw[i] = bswap(w[i]);
 }
 
-// Producer: W[t] + K[t] for t = 0..63 into one LDS slot, [quad][lane].
-__device__ __forceinline__ void sha_schedule(uint32_t w[16], u32x4 (*slot)[kShaColumns], int lane) {
+// Producer: W[t] + K[t] for t = 0..63 into column `column` of one LDS slot, [quad][column].
+template <int kColumns>
+__device__ __forceinline__ void sha_schedule(uint32_t w[16], u32x4 (*slot)[kColumns], int column) {
 #pragma unroll
     for (int q = 0; q < kShaBlockQuads; ++q) {
         uint32_t v[4];
@@ -1542,16 +1541,17 @@ __device__ __forceinline__ void sha_schedule(uint32_t w[16], u32x4 (*slot)[kShaC
             }
             v[i] = wt + kSha[t];
         }
-        slot[q][lane] = u32x4{v[0], v[1], v[2], v[3]};
+        slot[q][column] = u32x4{v[0], v[1], v[2], v[3]};
     }
 }
 
-// Round waves: two lanes per record.  Within each 8-lane half row, lanes 0-3
-// are "e-lanes" holding (e, f, g, h) and lanes 4-7 "a-lanes" holding (a, b,
-// c, d); e-lane i and a-lane 7 - i hold one record (DPP row_half_mirror
-// swaps them).  Both halves run one instruction stream on registers X0..X3,
-// the a-half two rounds behind: in slot t the e-lanes do round t and the
-// a-lanes round t - 2.  A slot computes
+// Round waves: within each 8-lane half row, lanes 0-3 are "e-lanes" holding
+// (e, f, g, h) and lanes 4-7 "a-lanes" holding (a, b, c, d); e-lane i and
+// a-lane 7 - i belong to one record (DPP row_half_mirror swaps them).  In the
+// two-lane form the half row holds four records; in the quad form it holds one,
+// whose e-lanes (and a-lanes) hold the same registers.  Both halves run one
+// instruction stream on registers X0..X3, the a-half two rounds behind: in
+// slot t the e-lanes do round t and the a-lanes round t - 2.  A slot computes
 //   W = (X3 ^ m) + K + partner's X1                   h + W[t]+K[t] + d | e' - d
 //   S = rotr(X0, r1) ^ rotr(X0, r2) ^ rotr(X0, r3)    Sigma1(e) | Sigma0(a)
 //   u = m ? ~(X0 ^ X1) : X0;  C = u ? X1 : X2         Ch(e,f,g) | Maj(a,b,c)
@@ -1560,17 +1560,35 @@ __device__ __forceinline__ void sha_schedule(uint32_t w[16], u32x4 (*slot)[kShaC
 // (Maj(a,b,c) = ~(a^b) ? b : c bitwise; ~d + 1 = -d).  With the two-round
 // lag the partner's X1 is what each half needs: the a-lanes' X1 is a of
 // round t - 4, the e-lanes' d; the e-lanes' X1 is e' of round t - 2, the
-// round the a-lanes are on.  So one DPP add serves both halves, it reads a
-// register written two slots before, and a slot is 9 VALU whose only chain
-// is the rotations (or Ch/Maj) into one add3.  (Both halves on the same
-// round need a DPP add on the chain and a second one for d: 11 issue slots
-// a round against 9.)
+// round the a-lanes are on.  So one DPP add serves both halves, and it reads a
+// register written two slots before.  (Both halves on the same round need a
+// DPP add on the chain and a second one for d: 11 issue slots a round.)
+//
+// The two-lane form rotates three times and XORs once (4 of its 9 VALU).  In
+// the quad form each lane of a half's four rotates by one of the three amounts
+// (the fourth repeats the first), one v_alignbit_b32 for all three rotations,
+// and two DPP XORs add the other two lanes' (3 of its 8 VALU).
+//
+// Measured, 512 records of 2.25 MiB in one launch: 43.7 ms for the two-lane
+// form as the compiler scheduled it (44.5 cycles a slot at 2.4 GHz), 41.5
+// cycles in assembly, 35.5-35.9 ms (36.1-36.5 cycles) for the quad form; 512
+// records of 288 KiB 5.47 and 4.48 ms.  What bounds it: 534 VALU a block at 4
+// cycles (2,136 of about 2,325), then the 16 LDS reads.
 constexpr int kDppIdentity = 0xE4;    // quad_perm [0,1,2,3]: lane i reads itself
 constexpr int kDppHalfMirror = 0x141;  // lane i reads lane 7 - i of its half row
 constexpr int kEBanks = 0x5, kABanks = 0xA;
 
+// The quad form's DPP quad permutations: lanes 0, 1, 2 read (1, 2), (2, 0), (0, 1); lane 3, whose rotation is
+// lane 0's, reads (1, 2).
+constexpr int kDppQuadNext = 1 | 2 << 2 | 0 << 4 | 1 << 6;
+constexpr int kDppQuadAfter = 2 | 0 << 2 | 1 << 4 | 2 << 6;
+
 struct ShaHalf {
     uint32_t r1, r2, r3, m;
+};
+
+struct ShaQuarter {
+    uint32_t r, m;
 };
 
 __device__ __forceinline__ uint32_t rotr_v(uint32_t x, uint32_t n) { return __builtin_amdgcn_alignbit(x, x, n); }
@@ -1582,8 +1600,6 @@ template <int kCtrl, int kBanks>
 __device__ __forceinline__ uint32_t dpp_bits(uint32_t x) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), kCtrl, 0xF, kBanks, false));
 }
-// The partner's x.
-__device__ __forceinline__ uint32_t from_partner(uint32_t x) { return dpp_bits<kDppHalfMirror, 0xF>(x); }
 // The partner's x on e-lanes (from the a-lane), 0 on a-lanes; and the other way round.
 __device__ __forceinline__ uint32_t from_a_partner(uint32_t x) { return dpp_bits<kDppHalfMirror, kEBanks>(x); }
 __device__ __forceinline__ uint32_t from_e_partner(uint32_t x) { return dpp_bits<kDppHalfMirror, kABanks>(x); }
@@ -1591,11 +1607,7 @@ __device__ __forceinline__ uint32_t from_e_partner(uint32_t x) { return dpp_bits
 __device__ __forceinline__ uint32_t on_e_lanes(uint32_t x) { return dpp_bits<kDppIdentity, kEBanks>(x); }
 __device__ __forceinline__ uint32_t on_a_lanes(uint32_t x) { return dpp_bits<kDppIdentity, kABanks>(x); }
 
-__device__ __forceinline__ uint32_t quad_word(const u32x4& q, int t) {
-    return (t & 3) == 0 ? q.x : (t & 3) == 1 ? q.y : (t & 3) == 2 ? q.z : q.w;
-}
-
-// Two-lane state between slots: X0..X3 as above and the chaining value, held
+// State between slots: X0..X3 as above and the chaining value, held
 // as E (the e-lanes' words) and F (the a-lanes' words).
 struct ShaLanes {
     uint32_t x[4];
@@ -1606,25 +1618,22 @@ __device__ __forceinline__ uint32_t sha_sigma(uint32_t x0, const ShaHalf& k) {
     return xor3(rotr_v(x0, k.r1), rotr_v(x0, k.r2), rotr_v(x0, k.r3));
 }
 
+__device__ __forceinline__ uint32_t sha_sigma(uint32_t x0, const ShaQuarter& k) {
+    const uint32_t y = rotr_v(x0, k.r);
+    return xor3(y, dpp_bits<kDppQuadNext, 0xF>(y), dpp_bits<kDppQuadAfter, 0xF>(y));
+}
+
 // bitop3 tables index bits as (src0 << 2) | (src1 << 1) | src2.
-__device__ __forceinline__ uint32_t sha_choose(uint32_t x0, uint32_t x1, uint32_t x2, const ShaHalf& k) {
-    const uint32_t u = __builtin_amdgcn_bitop3_b32(x0, x1, k.m, 0xD2);  // m ? ~(x0 ^ x1) : x0
+__device__ __forceinline__ uint32_t sha_choose(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t m) {
+    const uint32_t u = __builtin_amdgcn_bitop3_b32(x0, x1, m, 0xD2);  // m ? ~(x0 ^ x1) : x0
     return __builtin_amdgcn_bitop3_b32(x1, x2, u, 0xE4);                // u ? x1 : x2
 }
 
 // One slot whose W has been summed but for S + C.
-__device__ __forceinline__ void sha_slot_finish(ShaLanes& l, uint32_t w, const ShaHalf& k) {
-    const uint32_t v = sha_sigma(l.x[0], k) + sha_choose(l.x[0], l.x[1], l.x[2], k) + w;
+template <class Lanes>
+__device__ __forceinline__ void sha_slot_finish(ShaLanes& l, uint32_t w, const Lanes& k) {
+    const uint32_t v = sha_sigma(l.x[0], k) + sha_choose(l.x[0], l.x[1], l.x[2], k.m) + w;
     l.x[3] = l.x[2]; l.x[2] = l.x[1]; l.x[1] = l.x[0]; l.x[0] = v;
-}
-
-// A slot inside a block: one DPP add for both halves.
-__device__ __forceinline__ void sha_slot(ShaLanes& l, uint32_t word, const ShaHalf& k) {
-    uint32_t w = (l.x[3] ^ k.m) + word;
-    opaque(w);
-    w = from_partner(l.x[1]) + w;
-    opaque(w);
-    sha_slot_finish(l, w, k);
 }
 
 // Slot 0 or 1 of a block: the e-lanes' rounds 0 and 1 of this block, the
@@ -1633,8 +1642,9 @@ __device__ __forceinline__ void sha_slot(ShaLanes& l, uint32_t word, const ShaHa
 // e-lanes' d is the a-lanes' X1 plus the chaining word not yet added (`fw`,
 // d then c), and the a-lanes' e' is the e-lanes' X1 before the feed-forward
 // (`unfed`: the slot before's X1 and X0).
+template <class Lanes>
 __device__ __forceinline__ void sha_slot_turn(ShaLanes& l, uint32_t word, uint32_t fw, uint32_t unfed,
-                                              const ShaHalf& k) {
+                                              const Lanes& k) {
     uint32_t w = (l.x[3] ^ k.m) + word;
     opaque(w);
     w = from_a_partner(l.x[1] + fw) + w;
@@ -1647,7 +1657,8 @@ __device__ __forceinline__ void sha_slot_turn(ShaLanes& l, uint32_t word, uint32
 // Between blocks: the e-lanes add their chaining words to X0..X3 and keep the
 // sums as the chaining words (a-lanes untouched); slots 0 and 1 finish the
 // previous block on the a-lanes, which then do the same with F.
-__device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint32_t word1, const ShaHalf& k) {
+template <class Lanes>
+__device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint32_t word1, const Lanes& k) {
     const uint32_t unfed0 = l.x[0], unfed1 = l.x[1];
 #pragma unroll
     for (int i = 0; i < 4; ++i) l.e[i] = l.x[i] = l.x[i] + on_e_lanes(l.e[i]);
@@ -1657,46 +1668,152 @@ __device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint
     for (int i = 0; i < 4; ++i) l.f[i] = l.x[i] = l.x[i] + on_a_lanes(l.f[i]);
 }
 
-// The W+K words come from LDS in batches of four 16-byte quads (16 rounds),
-// each batch read a whole batch ahead of its use and waited for with one
-// s_waitcnt: a wait costs a wave about 7 cycles however little it waits, so
-// one wait for 16 rounds rather than one for every 4.  A scheduling barrier
-// after the reads keeps them where they are issued; left to itself the
-// compiler sinks them to their first use, a batch later.
-constexpr int kShaBatch = 4;                                 // quads a batch
-constexpr int kShaBatches = kShaBlockQuads / kShaBatch;      // batches a block
-constexpr unsigned kWaitLds = 0xC07F;                        // s_waitcnt lgkmcnt(0)
-
-__device__ __forceinline__ void sha_read_batch(u32x4 dst[kShaBatch], const u32x4 (*slot)[kShaColumns], int batch,
-                                               int column) {
-#pragma unroll
-    for (int j = 0; j < kShaBatch; ++j) dst[j] = slot[kShaBatch * batch + j][column];
-    __builtin_amdgcn_sched_barrier(0);
-}
+// A block's 64 slots, in assembly: the instructions, their order and their
+// addresses are the rate.  A VALU instruction takes 4 cycles of the wave's
+// SIMD, but an 8-byte one (every VOP3 and DPP instruction) whose address is 4
+// modulo 8 takes 5 (measured on one wave: a quad slot of eight such
+// instructions 32.5 cycles on 8-byte boundaries, 40.6 off them, whatever the
+// registers and the order within the slot), and every s_nop takes an issue
+// slot of its own.  The compiler, given the same operations, put two s_nop a
+// slot around the barriers that keep its adds in order and let its 4-byte
+// instructions shift the rest: 44.5 cycles a two-lane slot, where nine
+// instructions need 36.  So the block starts on an 8-byte boundary and its
+// 4-byte instructions come in pairs (the last, a wait, ends it).
+//
+// W + K words: the block's 64 in v64-v127 and the next block's in v128-v191,
+// or the other way round (kOdd).  The next block's sixteen ds_read_b128 go out
+// in two groups of eight and are waited for at the end, so no load is in
+// flight outside the statement.  Beside its own 4 cycles a read costs the wave
+// about 8 wherever VALU and LDS instructions alternate (on one wave, 16 reads
+// a block one by one 184 cycles, in fours 88); of the groupings, eight and
+// eight ran fastest (36.2 cycles a slot on the 8k session, two by two 36.8,
+// all sixteen 37.2, which then queue for the LDS).
+//
+// DPP reads a register at least two instructions after its write (the ISA's
+// two wait states), by the order within the macros: X1's last write is in the
+// slot before at the latest; a quad slot's rotation, `a`, is three
+// instructions before its first DPP XOR, and so is `t` before the turn's.
+//
+// The turn (slots 0 and 1) is sha_block_turn's: the e-lanes feed forward first
+// (bank_mask 0x5), the a-lanes after slot 1 (0xa).
+#define SHA_ALL " row_mask:0xf bank_mask:0xf\n"
+#define SHA_ON_E " row_mask:0xf bank_mask:0x5\n"
+#define SHA_ON_A " row_mask:0xf bank_mask:0xa\n"
+#define SHA_PARTNER(X1, X3) "v_add_u32_dpp " X3 ", " X1 ", " X3 " row_half_mirror" SHA_ALL
+#define SHA_TWO(X0, X1, X2, X3, W, BEFORE, PARTNER)                   \
+    "v_alignbit_b32 %[a], " X0 ", " X0 ", %[r1]\n"                    \
+    "v_alignbit_b32 %[b], " X0 ", " X0 ", %[r2]\n"                    \
+    "v_alignbit_b32 %[c], " X0 ", " X0 ", %[r3]\n" BEFORE             \
+    "v_xad_u32 " X3 ", " X3 ", %[m], " W "\n"                         \
+    "v_bitop3_b32 %[a], %[a], %[b], %[c] bitop3:0x96\n"               \
+    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n" PARTNER   \
+    "v_bitop3_b32 %[b], " X1 ", " X2 ", %[b] bitop3:0xe4\n"           \
+    "v_add3_u32 " X3 ", %[a], %[b], " X3 "\n"
+#define SHA_QUAD(X0, X1, X2, X3, W, BEFORE, PARTNER)                  \
+    "v_alignbit_b32 %[a], " X0 ", " X0 ", %[r1]\n"                    \
+    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n" BEFORE    \
+    "v_xad_u32 " X3 ", " X3 ", %[m], " W "\n"                         \
+    "v_xor_b32_dpp %[c], %[a], %[a] quad_perm:[1,2,0,1]" SHA_ALL      \
+    "v_bitop3_b32 %[b], " X1 ", " X2 ", %[b] bitop3:0xe4\n" PARTNER   \
+    "v_xor_b32_dpp %[c], %[a], %[c] quad_perm:[2,0,1,2]" SHA_ALL      \
+    "v_add3_u32 " X3 ", %[c], %[b], " X3 "\n"
+#define SHA_SLOT(S, X0, X1, X2, X3, W) S(X0, X1, X2, X3, W, "", SHA_PARTNER(X1, X3))
+#define SHA_SLOT_TURN(S, X0, X1, X2, X3, W, FW, UNFED)                \
+    S(X0, X1, X2, X3, W, "v_add_u32_e64 %[t], " FW ", " X1 "\n",      \
+      "v_add_u32_dpp " X3 ", %[t], " X3 " row_half_mirror" SHA_ON_E   \
+      "v_add_u32_dpp " X3 ", " UNFED ", " X3 " row_half_mirror" SHA_ON_A)
+#define SHA_WORD(I) "v[%[words]+" I "]"
+#define SHA_FOUR(S, W0, W1, W2, W3)                                   \
+    SHA_SLOT(S, "%[x0]", "%[x1]", "%[x2]", "%[x3]", W0)               \
+    SHA_SLOT(S, "%[x3]", "%[x0]", "%[x1]", "%[x2]", W1)               \
+    SHA_SLOT(S, "%[x2]", "%[x3]", "%[x0]", "%[x1]", W2)               \
+    SHA_SLOT(S, "%[x1]", "%[x2]", "%[x3]", "%[x0]", W3)
+#define SHA_FEED(BANKS, H, X) "v_add_u32_dpp " X ", " H ", " X " quad_perm:[0,1,2,3]" BANKS
+#define SHA_TURN_FOUR(S, W0, W1, W2, W3)                              \
+    "v_mov_b32_e32 %[u0], %[x0]\nv_mov_b32_e32 %[u1], %[x1]\n"        \
+    SHA_FEED(SHA_ON_E, "%[e0]", "%[x0]") SHA_FEED(SHA_ON_E, "%[e1]", "%[x1]") \
+    SHA_FEED(SHA_ON_E, "%[e2]", "%[x2]") SHA_FEED(SHA_ON_E, "%[e3]", "%[x3]") \
+    "v_mov_b32_e32 %[e0], %[x0]\nv_mov_b32_e32 %[e1], %[x1]\n"        \
+    "v_mov_b32_e32 %[e2], %[x2]\nv_mov_b32_e32 %[e3], %[x3]\n"        \
+    SHA_SLOT_TURN(S, "%[x0]", "%[x1]", "%[x2]", "%[x3]", W0, "%[f3]", "%[u1]") \
+    SHA_SLOT_TURN(S, "%[x3]", "%[x0]", "%[x1]", "%[x2]", W1, "%[f2]", "%[u0]") \
+    SHA_FEED(SHA_ON_A, "%[f0]", "%[x2]") SHA_FEED(SHA_ON_A, "%[f1]", "%[x3]") \
+    SHA_FEED(SHA_ON_A, "%[f2]", "%[x0]") SHA_FEED(SHA_ON_A, "%[f3]", "%[x1]") \
+    "v_mov_b32_e32 %[f0], %[x2]\nv_mov_b32_e32 %[f1], %[x3]\n"        \
+    "v_mov_b32_e32 %[f2], %[x0]\nv_mov_b32_e32 %[f3], %[x1]\n"        \
+    SHA_SLOT(S, "%[x2]", "%[x3]", "%[x0]", "%[x1]", W2)               \
+    SHA_SLOT(S, "%[x1]", "%[x2]", "%[x3]", "%[x0]", W3)
+// The next block's quads Q and Q + 1 of words, then four slots.
+#define SHA_READ(Q) "ds_read_b128 v[%[ahead]+4*(" Q "):%[ahead]+4*(" Q ")+3], %[next] offset:%[pitch]*(" Q ")+%[slot]\n"
+#define SHA_READ_TWO(Q) SHA_READ(Q) SHA_READ(Q "+1")
+#define SHA_GROUP(S, FOUR, I) FOUR(S, SHA_WORD(I), SHA_WORD(I "+1"), SHA_WORD(I "+2"), SHA_WORD(I "+3"))
+#define SHA_SIXTEEN(S, FIRST, I)                                      \
+    SHA_GROUP(S, FIRST, I) SHA_GROUP(S, SHA_FOUR, I "+4") SHA_GROUP(S, SHA_FOUR, I "+8") SHA_GROUP(S, SHA_FOUR, I "+12")
+#define SHA_READ_EIGHT(Q)                                             \
+    SHA_READ(Q) SHA_READ(Q "+1") SHA_READ(Q "+2") SHA_READ(Q "+3") SHA_READ(Q "+4") SHA_READ(Q "+5") SHA_READ(Q "+6") \
+    SHA_READ(Q "+7")
+#define SHA_BLOCK(S)                                                  \
+    ".p2align 3\n"                                                    \
+    SHA_READ_EIGHT("0") SHA_SIXTEEN(S, SHA_TURN_FOUR, "0")            \
+    SHA_READ_EIGHT("8") SHA_SIXTEEN(S, SHA_FOUR, "16")                \
+    SHA_SIXTEEN(S, SHA_FOUR, "32") SHA_SIXTEEN(S, SHA_FOUR, "48")     \
+    "s_waitcnt lgkmcnt(0)\n"
+#define SHA_BLOCK_STATE                                               \
+    [x0] "+v"(l.x[0]), [x1] "+v"(l.x[1]), [x2] "+v"(l.x[2]), [x3] "+v"(l.x[3]), [e0] "+v"(l.e[0]),               \
+        [e1] "+v"(l.e[1]), [e2] "+v"(l.e[2]), [e3] "+v"(l.e[3]), [f0] "+v"(l.f[0]), [f1] "+v"(l.f[1]),           \
+        [f2] "+v"(l.f[2]), [f3] "+v"(l.f[3]), [a] "=&v"(a), [b] "=&v"(b), [c] "=&v"(c), [t] "=&v"(t),            \
+        [u0] "=&v"(u0), [u1] "=&v"(u1)
+#define SHA_WORDS_64(MODE, Q)                                                                                     \
+    MODE "{v[64:67]}"(Q[0]), MODE "{v[68:71]}"(Q[1]), MODE "{v[72:75]}"(Q[2]), MODE "{v[76:79]}"(Q[3]),          \
+        MODE "{v[80:83]}"(Q[4]), MODE "{v[84:87]}"(Q[5]), MODE "{v[88:91]}"(Q[6]), MODE "{v[92:95]}"(Q[7]),      \
+        MODE "{v[96:99]}"(Q[8]), MODE "{v[100:103]}"(Q[9]), MODE "{v[104:107]}"(Q[10]),                          \
+        MODE "{v[108:111]}"(Q[11]), MODE "{v[112:115]}"(Q[12]), MODE "{v[116:119]}"(Q[13]),                      \
+        MODE "{v[120:123]}"(Q[14]), MODE "{v[124:127]}"(Q[15])
+#define SHA_WORDS_128(MODE, Q)                                                                                    \
+    MODE "{v[128:131]}"(Q[0]), MODE "{v[132:135]}"(Q[1]), MODE "{v[136:139]}"(Q[2]), MODE "{v[140:143]}"(Q[3]),  \
+        MODE "{v[144:147]}"(Q[4]), MODE "{v[148:151]}"(Q[5]), MODE "{v[152:155]}"(Q[6]),                         \
+        MODE "{v[156:159]}"(Q[7]), MODE "{v[160:163]}"(Q[8]), MODE "{v[164:167]}"(Q[9]),                         \
+        MODE "{v[168:171]}"(Q[10]), MODE "{v[172:175]}"(Q[11]), MODE "{v[176:179]}"(Q[12]),                      \
+        MODE "{v[180:183]}"(Q[13]), MODE "{v[184:187]}"(Q[14]), MODE "{v[188:191]}"(Q[15])
+#define SHA_ASM(S, ...)                                                                                           \
+    if (kOdd)                                                                                                     \
+        asm volatile(SHA_BLOCK(S) : SHA_BLOCK_STATE, SHA_WORDS_64("=&", ahead)                                    \
+                     : SHA_WORDS_128("", words), [words] "n"(128), [ahead] "n"(64), [next] "v"(next),             \
+                       [pitch] "n"(kPitch), [slot] "n"(kSlot), [m] "v"(k.m), __VA_ARGS__ : "memory");             \
+    else                                                                                                          \
+        asm volatile(SHA_BLOCK(S) : SHA_BLOCK_STATE, SHA_WORDS_128("=&", ahead)                                   \
+                     : SHA_WORDS_64("", words), [words] "n"(64), [ahead] "n"(128), [next] "v"(next),              \
+                       [pitch] "n"(kPitch), [slot] "n"(kSlot), [m] "v"(k.m), __VA_ARGS__ : "memory")
 
 // One block.  On entry the e-lanes hold the state after the previous block's
-// round 63 and the a-lanes after its round 61 (see sha_block_turn), and q[0]
-// holds this block's first W+K batch, not yet waited for; q[1] is free.  With
-// kNext the first batch of `next` is read during the last batch, into q[0].
-template <bool kNext>
-__device__ __forceinline__ void sha_block(ShaLanes& l, u32x4 (&q)[2][kShaBatch], const u32x4 (*slot)[kShaColumns],
-                                          const u32x4 (*next)[kShaColumns], int column, const ShaHalf& k) {
-#pragma unroll
-    for (int b = 0; b < kShaBatches; ++b) {
-        __builtin_amdgcn_s_waitcnt(kWaitLds);
-        if (b + 1 < kShaBatches)
-            sha_read_batch(q[(b + 1) & 1], slot, b + 1, column);
-        else if (kNext)
-            sha_read_batch(q[(b + 1) & 1], next, 0, column);
-        const u32x4* cur = q[b & 1];
-#pragma unroll
-        for (int t = 16 * b; t < 16 * b + 16; ++t) {
-            if (t == 0)
-                sha_block_turn(l, quad_word(cur[0], 0), quad_word(cur[0], 1), k);
-            else if (t > 1)
-                sha_slot(l, quad_word(cur[(t >> 2) & 3], t), k);
-        }
-    }
+// round 63 and the a-lanes after its round 61 (see sha_block_turn), and `words`
+// this block's words; on exit `ahead` holds the next block's, read from LDS
+// byte address next + kSlot, kPitch bytes from one quad of words to the next.
+template <int kPitch, int kSlot, bool kOdd>
+__device__ __forceinline__ void sha_block(ShaLanes& l, const u32x4 (&words)[kShaBlockQuads],
+                                          u32x4 (&ahead)[kShaBlockQuads], uint32_t next, const ShaHalf& k) {
+    uint32_t a, b, c, t, u0, u1;
+    SHA_ASM(SHA_TWO, [r1] "v"(k.r1), [r2] "v"(k.r2), [r3] "v"(k.r3));
+}
+
+template <int kPitch, int kSlot, bool kOdd>
+__device__ __forceinline__ void sha_block(ShaLanes& l, const u32x4 (&words)[kShaBlockQuads],
+                                          u32x4 (&ahead)[kShaBlockQuads], uint32_t next, const ShaQuarter& k) {
+    uint32_t a, b, c, t, u0, u1;
+    SHA_ASM(SHA_QUAD, [r1] "v"(k.r));
+}
+
+// Blocks kFirst on of a step whose LDS slots start at `at` (of `count` blocks), then the first words of the
+// next step's, at `next`.
+template <int kPitch, int kStep, int kFirst, class Lanes>
+__device__ __forceinline__ void sha_blocks(ShaLanes& l, u32x4 (&even)[kShaBlockQuads], u32x4 (&odd)[kShaBlockQuads],
+                                           uint32_t at, uint32_t next, uint32_t count, const Lanes& k) {
+    static_assert(kStep % 2 == 0, "a step ends on the words it began with");
+    if (kFirst >= count) return;  // wave-uniform
+    constexpr bool kOdd = kFirst % 2;
+    constexpr int kSlot = kFirst + 1 < kStep ? (kFirst + 1) * kShaBlockQuads * kPitch : 0;
+    sha_block<kPitch, kSlot, kOdd>(l, kOdd ? odd : even, kOdd ? even : odd, kSlot ? at : next, k);
+    if constexpr (kFirst + 1 < kStep) sha_blocks<kPitch, kStep, kFirst + 1>(l, even, odd, at, next, count, k);
 }
 
 // The lanes' state before the first block of a launch, from chaining value
@@ -1707,10 +1824,11 @@ __device__ __forceinline__ void sha_block(ShaLanes& l, u32x4 (&q)[2][kShaBatch],
 // + f - y3 and slot 1 Sigma0(b) + Maj(b, c, d) + e - y2, e and f being the
 // partner's X0 and X1 before the (here empty) feed-forward.  After them the
 // a-lanes hold (a, b, c, d).
-__device__ __forceinline__ ShaLanes sha_lanes_start(const uint32_t h[4], bool a_lane, const ShaHalf& k) {
+template <class Lanes>
+__device__ __forceinline__ ShaLanes sha_lanes_start(const uint32_t h[4], bool a_lane, const Lanes& k) {
     ShaLanes l;
-    const uint32_t y2 = sha_sigma(h[1], k) + sha_choose(h[1], h[2], h[3], k) + from_e_partner(h[0]) - h[0];
-    const uint32_t y3 = sha_sigma(h[2], k) + sha_choose(h[2], h[3], y2, k) + from_e_partner(h[1]) - h[1];
+    const uint32_t y2 = sha_sigma(h[1], k) + sha_choose(h[1], h[2], h[3], k.m) + from_e_partner(h[0]) - h[0];
+    const uint32_t y3 = sha_sigma(h[2], k) + sha_choose(h[2], h[3], y2, k.m) + from_e_partner(h[1]) - h[1];
     l.x[0] = a_lane ? h[2] : h[0];
     l.x[1] = a_lane ? h[3] : h[1];
     l.x[2] = a_lane ? y2 : h[2];
@@ -1723,108 +1841,168 @@ __device__ __forceinline__ ShaLanes sha_lanes_start(const uint32_t h[4], bool a_
 // After the last block: the e-lanes feed forward, the a-lanes run their
 // rounds 62 and 63 (K = 1) and feed forward; the chaining value is E on
 // e-lanes, F on a-lanes.
-__device__ __forceinline__ void sha_lanes_finish(ShaLanes& l, bool a_lane, const ShaHalf& k, uint32_t h[4]) {
+template <class Lanes>
+__device__ __forceinline__ void sha_lanes_finish(ShaLanes& l, bool a_lane, const Lanes& k, uint32_t h[4]) {
     sha_block_turn(l, 1u, 1u, k);
 #pragma unroll
     for (int i = 0; i < 4; ++i) h[i] = a_lane ? l.f[i] : l.e[i];
 }
 
-constexpr int kShaRoundWaves = 2;                  // round waves per workgroup, 32 records each
-constexpr int kShaProducers = 2;                   // message-schedule waves, alternate blocks of a step
-constexpr int kShaRecords = 32 * kShaRoundWaves;   // records per workgroup
-constexpr int kShaThreads = 64 * (kShaRoundWaves + kShaProducers);  // the round waves, then the producers
-constexpr int kShaStep = 4;  // blocks per barrier; the producers fill one half while the rounds read the other
-constexpr int kShaProducerBlocks = kShaStep / kShaProducers;  // blocks of a step per producer
+// The two forms' shapes.  A workgroup is kRounds round waves and kProducers
+// producer waves, four in all; kRecords records, kWaveRecords a round wave.  A
+// producer pass expands one block of every record (64 lanes, 64 records) or
+// two (32 lanes a block).  Blocks come in steps of kStep, one barrier a step:
+// the producers write step s + 2 into one of three buffers while the round
+// waves read step s, so the round waves read the next step's first words
+// before the barrier.  A producer loads a block 8 blocks ahead of its
+// expansion (about 7 us): beside a restore kernel's reads of host memory,
+// loads issued 4 blocks ahead came back late and the round waves waited at the
+// barrier (58 cycles a round against 45 at the time).
+struct ShaTwoLane {
+    static constexpr int kRounds = 2, kProducers = 2, kWaveRecords = 32, kStep = 2, kProducerLanes = 64;
+    using Lanes = ShaHalf;
+    __device__ static Lanes lanes(bool a_lane, int) {
+        return a_lane ? ShaHalf{2, 13, 22, ~0u} : ShaHalf{6, 11, 25, 0u};
+    }
+    // e-lane i and a-lane 7 - i of each half row share a record.
+    __device__ static int record(int lane, bool a_lane) {
+        return (lane >> 3) * 4 + (a_lane ? 3 - (lane & 3) : (lane & 3));
+    }
+    __device__ static bool writes(int) { return true; }
+};
 
-// A producer's step for block `blk` (of blocks below `end`): expand the words
-// loaded for it, then start the loads of block blk + kShaAheadSteps *
-// kShaStep into the same registers.  A producer keeps kShaAheadSteps register
-// sets per block of a step, so each block's loads are in flight for two whole
-// steps (about 10 us) before its expansion: beside a restore kernel's reads
-// of host memory, loads issued one step ahead came back late and the round
-// waves waited at the step barrier (58 cycles a round against 45).
-constexpr int kShaAheadSteps = 2;
+struct ShaQuad {
+    static constexpr int kRounds = 3, kProducers = 1, kWaveRecords = 8, kStep = 4, kProducerLanes = 32;
+    using Lanes = ShaQuarter;
+    __device__ static Lanes lanes(bool a_lane, int lane) {
+        const int j = lane & 3;
+        return a_lane ? ShaQuarter{j == 1 ? 13u : j == 2 ? 22u : 2u, ~0u}
+                      : ShaQuarter{j == 1 ? 11u : j == 2 ? 25u : 6u, 0u};
+    }
+    __device__ static int record(int lane, bool) { return lane >> 3; }
+    __device__ static bool writes(int lane) { return (lane & 3) == 0; }  // of the four lanes' equal copies
+};
 
-template <bool kAligned>
-__device__ __forceinline__ void sha_produce(const uint8_t* __restrict__ p, uint64_t record_bytes, uint64_t whole,
-                                            int nfinal, uint64_t end, uint64_t blk, uint32_t raw[16],
-                                            u32x4 (*slot)[kShaColumns], int lane) {
+constexpr int kShaThreads = 256;
+constexpr int kShaBuffers = 3;
+constexpr int kShaAheadBlocks = 8;
+
+template <class Form>
+struct ShaShape {
+    static constexpr int kRecords = Form::kRounds * Form::kWaveRecords;
+    static constexpr int kColumns = kRecords + 1;  // the records, then {1,1,1,1} for the a-lanes
+    static constexpr int kPitch = kColumns * 16;
+    static constexpr int kPassBlocks = 64 / Form::kProducerLanes;
+    static constexpr int kPasses = Form::kStep / kPassBlocks / Form::kProducers;  // per producer and step
+    static constexpr int kAhead = kShaAheadBlocks / Form::kStep;                  // steps of loads in flight
+    static_assert((Form::kRounds + Form::kProducers) * 64 == kShaThreads, "four waves");
+    static_assert(kPasses * Form::kProducers * kPassBlocks == Form::kStep, "a step splits evenly");
+    static_assert(2 * Form::kStep == 4 * kPassBlocks, "the four waves' first passes are two steps");
+    static_assert(kRecords <= Form::kProducerLanes, "a producer lane per record");
+    static_assert(Form::kStep * kShaBlockQuads * kPitch < 65536, "ds_read offsets");
+    using Schedule = u32x4[kShaBuffers][Form::kStep][kShaBlockQuads][kColumns];
+};
+
+// The step's barrier: this wave's LDS accesses are complete, its record loads may stay in flight.
+__device__ __forceinline__ void sha_step_barrier() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Expand the words loaded for a block into its slot.
+template <int kColumns>
+__device__ __forceinline__ void sha_expand(const uint32_t raw[16], u32x4 (*slot)[kColumns], int column) {
     uint32_t w[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) w[i] = bswap(raw[i]);
-    const uint64_t next = blk + kShaAheadSteps * kShaStep;
-    if (next < end) sha_message_raw<kAligned>(p, record_bytes, whole, nfinal, next, raw);
-    sha_schedule(w, slot, lane);
+    sha_schedule<kColumns>(w, slot, column);
 }
 
-// The register sets of the next two steps' blocks trade places.
-__device__ __forceinline__ void sha_rotate_sets(uint32_t (&raw)[kShaAheadSteps][kShaProducerBlocks][16]) {
-    static_assert(kShaAheadSteps == 2, "two sets");
-#pragma unroll
-    for (int j = 0; j < kShaProducerBlocks; ++j)
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const uint32_t t = raw[0][j][k];
-            raw[0][j][k] = raw[1][j][k];
-            raw[1][j][k] = t;
-        }
-}
-
-using ShaSchedule = u32x4[2][kShaStep][kShaBlockQuads][kShaColumns];
-
-// Blocks [b0, b1) of the chains of the `group`-th kShaRecords records.  b0 =
-// 0 starts from the FIPS 180-4 initial value, otherwise from `state` (8 words
-// per record, as a previous launch left them); b1 = nblocks writes the digest
-// to `out`, otherwise the chaining state back to `state`.  A whole hash in
-// one launch holds its stream (and any stream sharing its hardware queue) for
-// the whole chain; the host can run it as a series of shorter launches.
-template <bool kAligned>
-__device__ __forceinline__ void sha256_group(ShaSchedule& sched, const uint8_t* __restrict__ records,
-                                             uint64_t record_bytes, uint64_t pitch, int64_t n_records, uint64_t b0,
-                                             uint64_t b1, uint32_t* __restrict__ state, uint32_t* __restrict__ out,
+// Blocks [b0, b1) of the chains of the `group`-th kRecords records.  b0 = 0
+// starts from the FIPS 180-4 initial value, otherwise from `state` (8 words
+// per record, as a previous launch of either form left them); b1 = nblocks
+// writes the digest to `out`, otherwise the chaining state back to `state`.  A
+// whole hash in one launch holds its stream (and any stream sharing its
+// hardware queue) for the whole chain; the host can run it as a series of
+// shorter launches.
+template <class Form, bool kAligned>
+__device__ __forceinline__ void sha256_group(typename ShaShape<Form>::Schedule& sched,
+                                             const uint8_t* __restrict__ records, uint64_t record_bytes,
+                                             uint64_t pitch, int64_t n_records, uint64_t b0, uint64_t b1,
+                                             uint32_t* __restrict__ state, uint32_t* __restrict__ out,
                                              int64_t group) {
-    const int wave = threadIdx.x >> 6;
-    const bool producer = wave >= kShaRoundWaves;
-    const int part = wave - kShaRoundWaves;  // a producer's blocks of a step: part, part + kShaProducers, ...
+    using Shape = ShaShape<Form>;
+    constexpr int kStep = Form::kStep, kPassBlocks = Shape::kPassBlocks, kPasses = Shape::kPasses,
+                  kAhead = Shape::kAhead;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const bool a_lane = (lane >> 2) & 1;
-    // Record of this lane within the workgroup's kShaRecords (producer lanes past them idle).
-    // Round lanes: e-lane i and a-lane 7 - i of each 8-lane half row share a record.
-    const int rec = producer ? lane
-                             : wave * 32 + (lane >> 3) * 4 + (a_lane ? 3 - (lane & 3) : (lane & 3));
-    const int64_t r = group * kShaRecords + rec;
-    const bool live = rec < kShaRecords && r < n_records;
-    // Lanes past the last record hash record 0 (in bounds) and store nothing.
-    const uint8_t* p = records + (live ? r : 0) * pitch;
     const uint64_t whole = record_bytes / 64;
     const int nfinal = record_bytes - 64 * whole + 9 <= 64 ? 1 : 2;
     const uint64_t nblocks = whole + nfinal;
     const uint64_t span = b1 - b0;
-    const uint64_t steps = (span + kShaStep - 1) / kShaStep;
-    // raw[0]: the words of the producer's blocks of the next step to expand; raw[1]: of the step after.
-    uint32_t raw[kShaAheadSteps][kShaProducerBlocks][16];
-    if (producer) {
-        for (int i = lane + 64 * part; i < 2 * kShaStep * kShaBlockQuads; i += 64 * kShaProducers) {
-            const int slot = i / kShaBlockQuads;
-            sched[slot / kShaStep][slot % kShaStep][i % kShaBlockQuads][64] = u32x4{1u, 1u, 1u, 1u};
+    const uint64_t steps = (span + kStep - 1) / kStep;
+    // The record and the block of a pass that this lane expands; lanes past the last record expand record 0
+    // (in bounds), lanes past the workgroup's records nothing.
+    const int column = lane % Form::kProducerLanes, sub = lane / Form::kProducerLanes;
+    const bool expands = column < Shape::kRecords;
+    const int64_t mine = group * Shape::kRecords + column;
+    const uint8_t* source = records + (expands && mine < n_records ? mine : 0) * pitch;
+    const bool producer = wave >= Form::kRounds;
+    // The block of a step that a producer's pass j expands.
+    const auto pass_block = [&](int j) { return (wave - Form::kRounds + Form::kProducers * j) * kPassBlocks + sub; };
+    // raw[a]: the words of a producer's passes of step 2 + a, then of every kAhead-th step on, in flight.
+    uint32_t raw[kAhead][kPasses][16];
+    {
+        // The first two steps: one pass a wave, the producers' loads for the steps after them behind it.
+        const int i = wave * kPassBlocks + sub;
+        uint32_t first[16];
+        const bool some = expands && static_cast<uint64_t>(i) < span;
+        if (some) sha_message_raw<kAligned>(source, record_bytes, whole, nfinal, b0 + i, first);
+        if (producer) {
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a)
+#pragma unroll
+                for (int j = 0; j < kPasses; ++j) {
+                    const uint64_t blk = static_cast<uint64_t>((2 + a) * kStep + pass_block(j));
+                    if (expands && blk < span)
+                        sha_message_raw<kAligned>(source, record_bytes, whole, nfinal, b0 + blk, raw[a][j]);
+                }
         }
-#pragma unroll
-        for (int a = 0; a < kShaAheadSteps; ++a)
-#pragma unroll
-            for (int j = 0; j < kShaProducerBlocks; ++j) {
-                const uint64_t i = static_cast<uint64_t>(a * kShaStep + part + kShaProducers * j);
-                if (i < span) sha_message_raw<kAligned>(p, record_bytes, whole, nfinal, b0 + i, raw[a][j]);
-            }
-#pragma unroll
-        for (int j = 0; j < kShaProducerBlocks; ++j) {
-            const int i = part + kShaProducers * j;
-            if (static_cast<uint64_t>(i) < span)
-                sha_produce<kAligned>(p, record_bytes, whole, nfinal, b1, b0 + i, raw[0][j], sched[0][i], lane);
-        }
-        sha_rotate_sets(raw);
+        if (some) sha_expand<Shape::kColumns>(first, sched[i / kStep][i % kStep], column);
+        for (int k = threadIdx.x; k < kShaBuffers * kStep * kShaBlockQuads; k += kShaThreads)
+            (&sched[0][0][0])[k][Shape::kRecords] = u32x4{1u, 1u, 1u, 1u};
     }
-    __syncthreads();
-    ShaHalf half = a_lane ? ShaHalf{2, 13, 22, ~0u} : ShaHalf{6, 11, 25, 0u};
+    sha_step_barrier();
+    if (producer) {
+        int buffer = 2;
+        for (uint64_t step = 0; step < steps; step += kAhead) {
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                if (step + a >= steps) break;  // wave-uniform
+#pragma unroll
+                for (int j = 0; j < kPasses; ++j) {
+                    const int i = pass_block(j);
+                    const uint64_t blk = (step + a + 2) * kStep + i;
+                    if (expands && blk < span) {
+                        sha_expand<Shape::kColumns>(raw[a][j], sched[buffer][i], column);
+                        if (blk + kShaAheadBlocks < span)
+                            sha_message_raw<kAligned>(source, record_bytes, whole, nfinal,
+                                                      b0 + blk + kShaAheadBlocks, raw[a][j]);
+                    }
+                }
+                buffer = buffer == kShaBuffers - 1 ? 0 : buffer + 1;
+                sha_step_barrier();
+            }
+        }
+        return;
+    }
+    const bool a_lane = (lane >> 2) & 1;
+    const int rec = wave * Form::kWaveRecords + Form::record(lane, a_lane);
+    const int64_t r = group * Shape::kRecords + rec;
+    const bool live = r < n_records;
+    typename Form::Lanes half = Form::lanes(a_lane, lane);
     opaque(half.m);
     uint32_t h[4];
     uint32_t* chain = state ? state + 8 * (live ? r : 0) + (a_lane ? 0 : 4) : nullptr;
@@ -1837,52 +2015,42 @@ __device__ __forceinline__ void sha256_group(ShaSchedule& sched, const uint8_t* 
         h[0] = 0x510e527f; h[1] = 0x9b05688c; h[2] = 0x1f83d9ab; h[3] = 0x5be0cd19;
     }
     ShaLanes l = sha_lanes_start(h, a_lane, half);
-    const int column = a_lane ? 64 : rec;
-    u32x4 q[2][kShaBatch];  // W+K batches, read into alternately
+    const int word_column = a_lane ? Shape::kRecords : rec;
+    // LDS byte addresses of this lane's column, a step's slots after another's around the three buffers.
+    using LdsWord = __attribute__((address_space(3))) u32x4;
+    const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsWord*)&sched[0][0][0][word_column]));
+    constexpr uint32_t kStepBytes = kStep * kShaBlockQuads * Shape::kPitch;
+    uint32_t at = base;
+    u32x4 even[kShaBlockQuads], odd[kShaBlockQuads];
+#pragma unroll
+    for (int i = 0; i < kShaBlockQuads; ++i) even[i] = sched[0][0][i][word_column];
     for (uint64_t step = 0; step < steps; ++step) {
-        const uint64_t first = b0 + step * kShaStep;
-        if (producer) {
-#pragma unroll
-            for (int j = 0; j < kShaProducerBlocks; ++j) {
-                const int i = part + kShaProducers * j;
-                if (first + kShaStep + i < b1)
-                    sha_produce<kAligned>(p, record_bytes, whole, nfinal, b1, first + kShaStep + i, raw[0][j],
-                                          sched[(step + 1) & 1][i], lane);
-            }
-            sha_rotate_sets(raw);
-        } else {
-            sha_read_batch(q[0], sched[step & 1][0], 0, column);
-#pragma unroll
-            for (int i = 0; i < kShaStep; ++i) {
-                if (first + i >= b1) break;
-                if (i + 1 < kShaStep)
-                    sha_block<true>(l, q, sched[step & 1][i], sched[step & 1][i + 1], column, half);
-                else
-                    sha_block<false>(l, q, sched[step & 1][i], nullptr, column, half);
-            }
-        }
-        __syncthreads();
+        const uint64_t left = span - step * kStep;
+        const uint32_t next = at == base + (kShaBuffers - 1) * kStepBytes ? base : at + kStepBytes;
+        // Past the last block the words read are never used.
+        sha_blocks<Shape::kPitch, kStep, 0>(l, even, odd, at, next,
+                                            left < kStep ? static_cast<uint32_t>(left) : kStep, half);
+        at = next;
+        sha_step_barrier();
     }
-    if (!producer) {
-        sha_lanes_finish(l, a_lane, half, h);
-        if (live) {
-            if (b1 == nblocks)
-                *reinterpret_cast<u32x4*>(out + 8 * r + (a_lane ? 0 : 4)) =
-                    u32x4{bswap(h[0]), bswap(h[1]), bswap(h[2]), bswap(h[3])};
-            else
-                *reinterpret_cast<u32x4*>(chain) = u32x4{h[0], h[1], h[2], h[3]};
-        }
+    sha_lanes_finish(l, a_lane, half, h);
+    if (live && Form::writes(lane)) {
+        if (b1 == nblocks)
+            *reinterpret_cast<u32x4*>(out + 8 * r + (a_lane ? 0 : 4)) =
+                u32x4{bswap(h[0]), bswap(h[1]), bswap(h[2]), bswap(h[3])};
+        else
+            *reinterpret_cast<u32x4*>(chain) = u32x4{h[0], h[1], h[2], h[3]};
     }
 }
 
-template <bool kAligned>
+template <class Form, bool kAligned>
 __global__ __launch_bounds__(kShaThreads) void sha256_kernel(const uint8_t* __restrict__ records,
                                                              uint64_t record_bytes, uint64_t pitch,
                                                              int64_t n_records, uint64_t b0, uint64_t b1,
                                                              uint32_t* __restrict__ state,
                                                              uint32_t* __restrict__ out) {
-    __shared__ ShaSchedule sched;
-    sha256_group<kAligned>(sched, records, record_bytes, pitch, n_records, b0, b1, state, out, blockIdx.x);
+    __shared__ typename ShaShape<Form>::Schedule sched;
+    sha256_group<Form, kAligned>(sched, records, record_bytes, pitch, n_records, b0, b1, state, out, blockIdx.x);
 }
 
 // Several independent ranges in one launch: range blockIdx.y, its blockIdx.x-th
@@ -1904,17 +2072,17 @@ struct ShaRanges {
     ShaRange r[kShaMaxRanges];
 };
 
-template <bool kAligned>
+template <class Form, bool kAligned>
 __global__ __launch_bounds__(kShaThreads) void sha256_ranges_kernel(ShaRanges ranges) {
-    __shared__ ShaSchedule sched;
+    __shared__ typename ShaShape<Form>::Schedule sched;
     const ShaRange& g = ranges.r[blockIdx.y];
-    if (static_cast<int64_t>(blockIdx.x) * kShaRecords >= g.n_records) return;  // the whole workgroup
-    sha256_group<kAligned>(sched, g.records, g.record_bytes, g.pitch, g.n_records, g.b0, g.b1, g.state, g.out,
-                           blockIdx.x);
+    if (static_cast<int64_t>(blockIdx.x) * ShaShape<Form>::kRecords >= g.n_records) return;  // the whole workgroup
+    sha256_group<Form, kAligned>(sched, g.records, g.record_bytes, g.pitch, g.n_records, g.b0, g.b1, g.state, g.out,
+                                 blockIdx.x);
 }
 
 // The round's own issue rate, measured: one wave runs `reps` slots of the
-// round waves' instruction sequence (sha_slot, both halves) on values seeded
+// two-lane form's instruction sequence (SHA_TWO, both halves) on values seeded
 // per lane, with no LDS, no waits and no barrier, between two reads of the
 // shader clock (s_memtime) and of the 100 MHz constant clock (s_memrealtime).
 // out[0] = shader cycles, out[1] = constant-clock ticks, out[2] = a checksum
@@ -1924,30 +2092,29 @@ constexpr int kShaProbeUnroll = 16;
 __global__ __launch_bounds__(64) void sha_round_probe_kernel(uint32_t seed, int reps, uint64_t* __restrict__ out) {
     const int lane = threadIdx.x;
     const bool a_lane = (lane >> 2) & 1;
-    ShaHalf half = a_lane ? ShaHalf{2, 13, 22, ~0u} : ShaHalf{6, 11, 25, 0u};
+    ShaHalf half = ShaTwoLane::lanes(a_lane, lane);
     opaque(half.m);
-    ShaLanes l;
+    uint32_t x[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        l.x[i] = seed * 0x9E3779B9u + static_cast<uint32_t>(lane * 4 + i) * 0x85EBCA6Bu;
-        l.e[i] = l.f[i] = 0;
-    }
-    uint32_t word = a_lane ? 1u : seed ^ 0x5A827999u;
-    opaque(word);
+    for (int i = 0; i < 4; ++i) x[i] = seed * 0x9E3779B9u + static_cast<uint32_t>(lane * 4 + i) * 0x85EBCA6Bu;
+    const uint32_t word = a_lane ? 1u : seed ^ 0x5A827999u;
     const int rounds = reps / kShaProbeUnroll;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) opaque(l.x[i]);
+    for (int i = 0; i < 4; ++i) opaque(x[i]);
     const uint64_t c0 = __builtin_amdgcn_s_memtime();
     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
     for (int r = 0; r < rounds; ++r) {
-#pragma unroll
-        for (int k = 0; k < kShaProbeUnroll; ++k) sha_slot(l, word, half);
+        uint32_t a, b, c;
+#define SHA_PROBE_FOUR SHA_FOUR(SHA_TWO, "%[w]", "%[w]", "%[w]", "%[w]")
+        asm volatile(".p2align 3\n" SHA_PROBE_FOUR SHA_PROBE_FOUR SHA_PROBE_FOUR SHA_PROBE_FOUR
+                     : [x0] "+v"(x[0]), [x1] "+v"(x[1]), [x2] "+v"(x[2]), [x3] "+v"(x[3]), [a] "=&v"(a),
+                       [b] "=&v"(b), [c] "=&v"(c)
+                     : [r1] "v"(half.r1), [r2] "v"(half.r2), [r3] "v"(half.r3), [m] "v"(half.m), [w] "v"(word));
+#undef SHA_PROBE_FOUR
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) opaque(l.x[i]);
     const uint64_t c1 = __builtin_amdgcn_s_memtime();
     const uint64_t t1 = __builtin_amdgcn_s_memrealtime();
-    uint32_t sum = l.x[0] ^ l.x[1] ^ l.x[2] ^ l.x[3];
+    uint32_t sum = x[0] ^ x[1] ^ x[2] ^ x[3];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum ^= __shfl_xor(sum, o);
     if (lane == 0) {
@@ -2287,8 +2454,23 @@ uint32_t* static_crc_workspace() {
 constexpr unsigned kCuLds = 160 * 1024;
 constexpr unsigned kCopyLdsFence = kCuLds;                                        // plain copies: no LDS of their own
 constexpr unsigned kCheckedLdsFence = kCuLds - sizeof(uint32_t) * kCheckedLdsWords;  // the checked copies' tables
-constexpr unsigned kShaLdsFence = kCuLds - sizeof(ShaSchedule);
-static_assert(sizeof(ShaSchedule) < kCuLds, "a SHA-256 workgroup fits a CU");
+template <class Form>
+constexpr unsigned kShaLdsFence = kCuLds - sizeof(typename ShaShape<Form>::Schedule);
+static_assert(sizeof(ShaShape<ShaTwoLane>::Schedule) < kCuLds && sizeof(ShaShape<ShaQuad>::Schedule) < kCuLds,
+              "a SHA-256 workgroup fits a CU");
+
+// The quad form while its workgroups (24 records each) take at most a quarter
+// of the chip's 256 CUs, the two-lane form (64 records each) for more records
+// at once: every workgroup holds its CU for the whole launch, and the CUs are
+// the engine's too.  Both forms' times are one record's chain, whatever the
+// number of records, until a form runs out of CUs (records of 288 KiB: 4.50 ms
+// for 1536 in the quad form, 5.1 ms for 2000 in the two-lane form).
+constexpr int64_t kShaQuadGroups = 64;
+
+template <class Form>
+int64_t sha_groups(int64_t n_records) {
+    return (n_records + ShaShape<Form>::kRecords - 1) / ShaShape<Form>::kRecords;
+}
 
 }  // namespace
 
@@ -2642,6 +2824,21 @@ void check_sha_range(const void* records, uint64_t record_bytes, int64_t n_recor
         throw std::runtime_error("SHA-256 output and state must be 16-byte aligned");
 }
 
+template <class Form>
+void launch_sha(const ShaRange& g, bool aligned, hipStream_t s) {
+    hipLaunchKernelGGL((aligned ? sha256_kernel<Form, true> : sha256_kernel<Form, false>),
+                       dim3(static_cast<unsigned>(sha_groups<Form>(g.n_records))), dim3(kShaThreads),
+                       kShaLdsFence<Form>, s, g.records, g.record_bytes, g.pitch, g.n_records, g.b0, g.b1, g.state,
+                       g.out);
+}
+
+template <class Form>
+void launch_sha_ranges(const ShaRanges& ranges, int used, int64_t groups, bool aligned, hipStream_t s) {
+    hipLaunchKernelGGL((aligned ? sha256_ranges_kernel<Form, true> : sha256_ranges_kernel<Form, false>),
+                       dim3(static_cast<unsigned>(groups), static_cast<unsigned>(used)), dim3(kShaThreads),
+                       kShaLdsFence<Form>, s, ranges);
+}
+
 }  // namespace
 
 extern "C" {
@@ -2656,7 +2853,7 @@ int kvsnap_sha256_ranges(int count, const uint64_t* records, const uint64_t* rec
             throw std::runtime_error("SHA-256 ranges need every table");
         ShaRanges ranges{};
         int used = 0;
-        int64_t groups = 0;
+        int64_t two_lane = 0, quad = 0, quads = 0;
         bool aligned = true;
         for (int i = 0; i < count; ++i) {
             const auto* base = reinterpret_cast<const uint8_t*>(records[i]);
@@ -2667,16 +2864,17 @@ int kvsnap_sha256_ranges(int count, const uint64_t* records, const uint64_t* rec
             aligned = aligned && records[i] % 16 == 0 && record_pitches[i] % 16 == 0;
             ranges.r[used++] = ShaRange{base, record_bytes[i], record_pitches[i], n_records[i], first_blocks[i],
                                         end_blocks[i], state, reinterpret_cast<uint32_t*>(out)};
-            groups = std::max<int64_t>(groups, (n_records[i] + kShaRecords - 1) / kShaRecords);
+            two_lane = std::max(two_lane, sha_groups<ShaTwoLane>(n_records[i]));
+            quad = std::max(quad, sha_groups<ShaQuad>(n_records[i]));
+            quads += sha_groups<ShaQuad>(n_records[i]);
         }
         if (!used) return;
-        if (groups > (int64_t(1) << 30)) throw std::runtime_error("SHA-256: too many records");
+        if (two_lane > (int64_t(1) << 30)) throw std::runtime_error("SHA-256: too many records");
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-        const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(used));
-        if (aligned)
-            hipLaunchKernelGGL(sha256_ranges_kernel<true>, grid, dim3(kShaThreads), kShaLdsFence, s, ranges);
+        if (quads <= kShaQuadGroups)
+            launch_sha_ranges<ShaQuad>(ranges, used, quad, aligned, s);
         else
-            hipLaunchKernelGGL(sha256_ranges_kernel<false>, grid, dim3(kShaThreads), kShaLdsFence, s, ranges);
+            launch_sha_ranges<ShaTwoLane>(ranges, used, two_lane, aligned, s);
         check_launch("sha256 ranges");
     });
 }
@@ -2690,15 +2888,12 @@ int kvsnap_sha256_records_range(const void* records, uint64_t record_bytes, uint
         check_sha_range(records, record_bytes, n_records, first_block, end_block, state, out);
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
         const bool aligned = (reinterpret_cast<uintptr_t>(records) % 16 == 0) && (record_pitch % 16 == 0);
-        const unsigned grid = static_cast<unsigned>((n_records + kShaRecords - 1) / kShaRecords);
-        const auto* base = static_cast<const uint8_t*>(records);
-        auto* words = reinterpret_cast<uint32_t*>(out);
-        if (aligned)
-            hipLaunchKernelGGL(sha256_kernel<true>, dim3(grid), dim3(kShaThreads), kShaLdsFence, s, base, record_bytes,
-                               record_pitch, n_records, first_block, end_block, state, words);
+        const ShaRange range{static_cast<const uint8_t*>(records), record_bytes, record_pitch, n_records, first_block,
+                             end_block, state, reinterpret_cast<uint32_t*>(out)};
+        if (sha_groups<ShaQuad>(n_records) <= kShaQuadGroups)
+            launch_sha<ShaQuad>(range, aligned, s);
         else
-            hipLaunchKernelGGL(sha256_kernel<false>, dim3(grid), dim3(kShaThreads), kShaLdsFence, s, base, record_bytes,
-                               record_pitch, n_records, first_block, end_block, state, words);
+            launch_sha<ShaTwoLane>(range, aligned, s);
         check_launch("sha256");
     });
 }
