@@ -142,6 +142,19 @@ int kvsnap_scatter_blocks(const void* records, int64_t record_pitch, const int64
                           const int64_t* span_words, int64_t n_spans, int64_t min_span_bytes, int programs,
                           uintptr_t stream);
 
+/* At most 128 blocks between the cache and their records in one launch with no
+ * device table before it: `records` (addresses of packed records, pinned or
+ * device memory) and `blocks` are host arrays, read before the call returns.
+ * save != 0 writes the records, else the cache blocks.  tokens > 0 (a block's
+ * token slots, the outermost axis of every span): a save's last record keeps
+ * the first `filled` slots of each span, whose length / tokens is a multiple of
+ * 8 bytes, and the rest is written as zeros; tokens = filled = 0: every byte is
+ * copied.  min_span_bytes and programs are as for kvsnap_restore_blocks. */
+int kvsnap_copy_few(int save, const uint64_t* records, const int64_t* blocks, int64_t n_blocks,
+                    const int64_t* span_offsets, const int64_t* span_bases, const int64_t* span_pitches,
+                    const int64_t* span_words, int64_t n_spans, int64_t min_span_bytes, int64_t filled, int64_t tokens,
+                    int programs, uintptr_t stream);
+
 /* Copy nbytes from pinned host memory to device memory on `stream` (the DMA
  * engines, hipMemcpyAsync).  The restore's "dma" mode stages records with it
  * and then scatters them with kvsnap_scatter_blocks, so that a restore's

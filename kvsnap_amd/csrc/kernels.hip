@@ -260,6 +260,44 @@ __global__ __launch_bounds__(kRestoreThreads) void gather_to_kernel(
     }
 }
 
+// Few blocks between the cache and their records (pinned or device memory), in
+// one launch that needs nothing before it: the block ids and record addresses
+// ride in the kernel's arguments instead of a table copied to the device first
+// (16 us of host time and 10 of the stream's before the launch could start),
+// and a save's unfilled token slots are written as zeros on the way, where the
+// general path launches the zero kernel on staged records.  For layouts with
+// the token axis outermost in every span: the last record keeps the first
+// `filled` / `tokens` of each span.  A launch of up to kFewFreeBytes asks for
+// no LDS fence: it is over in 0.15 ms, and one that asked for whole CUs would
+// wait for them beside an engine's kernels.
+constexpr int kFewBlocks = 128;
+constexpr int64_t kFewFreeBytes = 8 << 20;
+
+struct FewBlocks {
+    int64_t block[kFewBlocks];
+    uint64_t record[kFewBlocks];
+};
+
+template <bool kSave>
+__global__ __launch_bounds__(kRestoreThreads) void copy_few_kernel(
+    const FewBlocks few, int64_t n_blocks, const int64_t* __restrict__ offs, const int64_t* __restrict__ bases,
+    const int64_t* __restrict__ pitches, const int64_t* __restrict__ words, int64_t n_spans, int lane_shift,
+    int64_t filled, int64_t tokens) {
+    const JobLanes jl = job_lanes<kRestoreThreads>(lane_shift);
+    const uint32_t spans = static_cast<uint32_t>(n_spans), jobs = static_cast<uint32_t>(n_blocks) * spans;
+    for (uint32_t job = blockIdx.x * jl.per_pass + jl.group; job < jobs; job += gridDim.x * jl.per_pass) {
+        const uint32_t b = job / spans, s = job - b * spans;
+        char* record = reinterpret_cast<char*>(few.record[b] + offs[s]);
+        char* cache = reinterpret_cast<char*>(bases[s] + few.block[b] * pitches[s]);
+        const int64_t length = words[s] * 8;
+        const int64_t keep = kSave && tokens && b + 1 == n_blocks ? length / tokens * filled : length;
+        copy_span<kRestoreUnroll>(kSave ? cache : record, kSave ? record : cache, keep, jl.lane, jl.lanes);
+        if (kSave)
+            for (int64_t i = keep + 8 * jl.lane; i < length; i += 8 * jl.lanes)
+                *reinterpret_cast<uint64_t*>(record + i) = 0;
+    }
+}
+
 // One wave that sleeps for `iters` rounds of s_sleep 127 (about 3.4 us each
 // at 2.4 GHz) and then ends: a fixed count, so every launch finishes.  The
 // data plane holds a stream with it for a few milliseconds to see which other
@@ -2700,6 +2738,33 @@ int kvsnap_gather_to_records(const int64_t* dests, const int64_t* blocks, int64_
                            reinterpret_cast<hipStream_t>(stream), dests, blocks, n_blocks, span_offsets, span_bases,
                            span_pitches, span_words, n_spans, shape.lane_shift);
         check_launch("gather to records");
+    });
+}
+
+int kvsnap_copy_few(int save, const uint64_t* records, const int64_t* blocks, int64_t n_blocks,
+                    const int64_t* span_offsets, const int64_t* span_bases, const int64_t* span_pitches,
+                    const int64_t* span_words, int64_t n_spans, int64_t min_span_bytes, int64_t filled, int64_t tokens,
+                    int programs, uintptr_t stream) {
+    return guard([&] {
+        if (n_blocks < 0 || n_blocks > kFewBlocks || n_spans < 0 || n_spans > (int64_t(1) << 20))
+            throw std::runtime_error("copy of few blocks: 0 to 128 blocks of at most 2^20 spans");
+        if (min_span_bytes > (int64_t(1) << 32)) min_span_bytes = int64_t(1) << 32;  // a shape hint, no more
+        if (filled < 0 || tokens < 0 || (tokens ? filled > tokens : filled))
+            throw std::runtime_error("copy of few blocks: more slots filled than a block has");
+        if (n_blocks == 0 || n_spans == 0) return;
+        if (!records || !blocks || !span_offsets || !span_bases || !span_pitches || !span_words)
+            throw std::runtime_error("copy of few blocks needs its host lists and device tables");
+        FewBlocks few{};
+        std::copy(blocks, blocks + n_blocks, few.block);
+        std::copy(records, records + n_blocks, few.record);
+        const CopyShape shape = copy_shape(kRestoreThreads, kRestoreUnroll, n_blocks * n_spans, min_span_bytes,
+                                           programs);
+        const unsigned fence = n_blocks * n_spans * min_span_bytes > kFewFreeBytes ? kCopyLdsFence : 0;
+        hipLaunchKernelGGL((save ? copy_few_kernel<true> : copy_few_kernel<false>), dim3(shape.grid),
+                           dim3(kRestoreThreads), fence, reinterpret_cast<hipStream_t>(stream), few, n_blocks,
+                           span_offsets, span_bases, span_pitches, span_words, n_spans, shape.lane_shift, filled,
+                           tokens);
+        check_launch("copy of few blocks");
     });
 }
 
