@@ -142,6 +142,16 @@ int kvsnap_scatter_blocks(const void* records, int64_t record_pitch, const int64
                           const int64_t* span_words, int64_t n_spans, int64_t min_span_bytes, int programs,
                           uintptr_t stream);
 
+/* SHA-256 (32 bytes each) and CRC32C of n records of record_bytes in host
+ * memory, on at most `threads` host threads (1 to 256; the caller's is one of
+ * them, the others end before the call does).  Needs a CPU with the SHA and
+ * SSE4.2 instructions: kvsnap_hash_records_available() is 1 there, else 0.  No
+ * GPU call is made.  (The reference hashes on host threads,
+ * kvsnap/connector/volatile.py:151.) */
+int kvsnap_hash_records_available(void);
+int kvsnap_hash_records(const uint64_t* records, uint64_t record_bytes, int64_t n_records, uint8_t* digests,
+                        uint32_t* crcs, int threads);
+
 /* At most 128 blocks between the cache and their records in one launch with no
  * device table before it: `records` (addresses of packed records, pinned or
  * device memory) and `blocks` are host arrays, read before the call returns.

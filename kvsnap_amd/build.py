@@ -2,7 +2,7 @@
 
     python -m kvsnap_amd.build
 
-``_native/libkvsnap_hip.so``  pinned pool + HIP kernels (hipcc, gfx950)
+``_native/libkvsnap_hip.so``  pinned pool + HIP kernels + host record hashes (hipcc, gfx950)
 ``_native/libkvsnap_io.so``   host CRC32C + pread/pwrite pool (g++)
 
 Both always rebuild when asked; the loaders only use what is already built.
@@ -53,7 +53,8 @@ def _atomic_output(target: Path) -> Path:
 
 def build_hip(target: Path = HIP_LIBRARY) -> Path:
     tmp = _atomic_output(target)
-    _run([_hipcc(), *HIPCC_FLAGS, "-o", str(tmp), str(CSRC / "kernels.hip"), str(CSRC / "pool.cpp")])
+    _run([_hipcc(), *HIPCC_FLAGS, "-o", str(tmp), str(CSRC / "kernels.hip"), str(CSRC / "pool.cpp"),
+          str(CSRC / "hash.cpp")])
     os.replace(tmp, target)
     return target
 

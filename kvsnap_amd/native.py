@@ -52,6 +52,8 @@ KERNEL_SIGNATURES = {
     "kvsnap_scatter_blocks": "int <- ptr i64 ptr i64 ptr ptr ptr ptr i64 i64 int stream",
     "kvsnap_gather_to_records": "int <- ptr ptr i64 ptr ptr ptr ptr i64 i64 int stream",
     "kvsnap_copy_few": "int <- int ptr ptr i64 ptr ptr ptr ptr i64 i64 i64 i64 int stream",
+    "kvsnap_hash_records_available": "int <-",
+    "kvsnap_hash_records": "int <- ptr u64 i64 ptr ptr int",
     "kvsnap_copy_to_device": "int <- ptr ptr size stream",
     "kvsnap_copy_to_host": "int <- ptr ptr size stream",
     "kvsnap_zero_regions": "int <- ptr ptr ptr i64 stream",

@@ -1,0 +1,35 @@
+"""Hashed saves of few records on the GPU plane: digests at hand when the save returns, equal to the oracle's."""
+import numpy as np
+import pytest
+import torch
+
+from kvsnap_amd import dataplane, synth
+from kvsnap_amd.native import kernel_library
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mode", ["staged", "direct"])
+@pytest.mark.parametrize("layout", ["vllm", "kv_split"])
+@pytest.mark.parametrize("n", [1, 2, 20, 65])
+def test_digests_equal_the_oracle(hip_library, oracle_lib, mode, layout, n):
+    caches, backing = synth.make_caches(4, 80, layout=layout)
+    plane = dataplane.TorchBlockDataPlane(caches, 16, 64 << 20, save_mode=mode)
+    try:
+        plane.warm_up()
+        keep = synth.fill(plane, n)
+        torch.cuda.synchronize()
+        hosted = plane._hash_threads(kernel_library(), n)
+        staged, digests, size = plane.pool.reserve(n * plane.block_bytes), [], plane.block_bytes
+        plane.save_gather(list(range(3, 3 + n)), [(staged, i * size) for i in range(n)], n * 16 - 5, digests=digests)
+        assert not hosted or digests[0].ready()
+        crcs, shas = oracle_lib.digest_records(staged.pointer, size, size, n, threads=4)
+        assert digests[0].result() == [(bytes(h).hex(), int(c)) for h, c in zip(shas, crcs)]
+        record = np.frombuffer(staged.read_range((n - 1) * size, size), dtype=np.uint8)
+        expected = record.copy()
+        oracle_lib.zero_tail(expected, plane.layers, 11)
+        assert np.array_equal(record, expected)
+        staged.close()
+        del keep
+    finally:
+        plane.close()
