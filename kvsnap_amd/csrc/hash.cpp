@@ -162,9 +162,10 @@ void hash_records(const uint64_t* records, uint64_t nbytes, int64_t n, uint8_t* 
     std::vector<std::thread> others;
     // A thread is worth starting (about 15 us) for 64 KiB of its own.
     const int64_t useful = std::min<int64_t>({threads, jobs, static_cast<int64_t>(nbytes * n >> 16)});
+    others.reserve(static_cast<size_t>(std::max<int64_t>(useful, 1)));
     try {
         for (int64_t i = 1; i < useful; ++i) others.emplace_back(work);
-    } catch (const std::system_error&) {
+    } catch (...) {
         // No more threads to be had: the ones there are, this one at least, do all the work.
     }
     work();
