@@ -24,8 +24,8 @@
 //
 // No MFMA anywhere: nothing on this path is a contraction.  The copies are
 // 16-byte-per-lane streams (4 or 8 dwordx4 loads in flight per lane), the CRC
-// is LDS table lookups combined in GF(2), and SHA-256 runs one record per two
-// lanes because the hash is a sequential chain within a record.
+// is LDS table lookups combined in GF(2), and SHA-256 gives a record two or
+// eight lanes because the hash is a sequential chain within a record.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -2502,7 +2502,7 @@ uint32_t* static_crc_workspace() {
 // can share their CU.  Beside a copy wave a SHA-256 round wave slows (range
 // launches took 2.5-3.5 ms beside the restore kernel, 1.8 ms alone); and an
 // engine's workgroup placed beside a SHA-256 workgroup gets the VALU issue
-// slots its round waves leave (they issue in about 84 % of them), so a
+// slots its round waves leave (they issue in about 90 % of them), so a
 // decode step whose workgroups are dealt evenly over the chip waits for the
 // ones on those CUs (the synthetic decode's median step went from 0.80 to
 // 0.75 ms beside hashed saves once the SHA-256 workgroups took whole CUs).

@@ -11,9 +11,10 @@ every block of every save (``README.md:795``: "Saves rehash every block").
 prepared record's shape (segments in block order; ``locations`` by blob id),
 with two changes on the data path:
 
-* the ids and CRC32Cs come from the GPU
-  (``TorchBlockDataPlane.save_gather(..., digests=[])``), computed from the
-  save's device staging while the D2H runs;
+* the ids and CRC32Cs come with the save
+  (``TorchBlockDataPlane.save_gather(..., digests=[])``), computed on the GPU
+  from its device staging while the D2H runs, or for few records on host
+  threads as they land;
 * ``save(..., previous=snapshot)`` gathers, copies and hashes only the blocks
   past the unchanged prefix (:func:`unchanged_prefix`): positions that hold
   the same block id as the previous snapshot of the session and were full
