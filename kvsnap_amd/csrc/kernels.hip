@@ -1745,10 +1745,14 @@ __device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint
 // eight ran fastest (36.2 cycles a slot on the 8k session, two by two 36.8,
 // all sixteen 37.2, which then queue for the LDS).
 //
-// DPP reads a register at least two instructions after its write (the ISA's
-// two wait states), by the order within the macros: X1's last write is in the
-// slot before at the latest; a quad slot's rotation, `a`, is three
-// instructions before its first DPP XOR, and so is `t` before the turn's.
+// Between a write of a register and a DPP instruction with it stand at least
+// two others (the ISA's two wait states, which the compiler does not look for
+// in here), whether it is the permuted source, the other one or the
+// destination, which masked lanes keep: between a slot's v_xad into X3 and the
+// partner's add, between the turn's two masked adds into X3 (FIRST, SECOND),
+// and between a quad slot's rotation, `a`, its first DPP XOR, `c`, and the
+// second.  X1 was written two slots before, and of the a-lanes' feeds the one
+// into slot 1's result comes last.
 //
 // The turn (slots 0 and 1) is sha_block_turn's: the e-lanes feed forward first
 // (bank_mask 0x5), the a-lanes after slot 1 (0xa).
@@ -1756,27 +1760,27 @@ __device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint
 #define SHA_ON_E " row_mask:0xf bank_mask:0x5\n"
 #define SHA_ON_A " row_mask:0xf bank_mask:0xa\n"
 #define SHA_PARTNER(X1, X3) "v_add_u32_dpp " X3 ", " X1 ", " X3 " row_half_mirror" SHA_ALL
-#define SHA_TWO(X0, X1, X2, X3, W, BEFORE, PARTNER)                   \
+#define SHA_TWO(X0, X1, X2, X3, W, BEFORE, FIRST, SECOND)             \
+    BEFORE "v_xad_u32 " X3 ", " X3 ", %[m], " W "\n"                  \
     "v_alignbit_b32 %[a], " X0 ", " X0 ", %[r1]\n"                    \
-    "v_alignbit_b32 %[b], " X0 ", " X0 ", %[r2]\n"                    \
-    "v_alignbit_b32 %[c], " X0 ", " X0 ", %[r3]\n" BEFORE             \
-    "v_xad_u32 " X3 ", " X3 ", %[m], " W "\n"                         \
-    "v_bitop3_b32 %[a], %[a], %[b], %[c] bitop3:0x96\n"               \
-    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n" PARTNER   \
+    "v_alignbit_b32 %[b], " X0 ", " X0 ", %[r2]\n" FIRST              \
+    "v_alignbit_b32 %[c], " X0 ", " X0 ", %[r3]\n"                    \
+    "v_bitop3_b32 %[a], %[a], %[b], %[c] bitop3:0x96\n" SECOND        \
+    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n"           \
     "v_bitop3_b32 %[b], " X1 ", " X2 ", %[b] bitop3:0xe4\n"           \
     "v_add3_u32 " X3 ", %[a], %[b], " X3 "\n"
-#define SHA_QUAD(X0, X1, X2, X3, W, BEFORE, PARTNER)                  \
-    "v_alignbit_b32 %[a], " X0 ", " X0 ", %[r1]\n"                    \
-    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n" BEFORE    \
+#define SHA_QUAD(X0, X1, X2, X3, W, BEFORE, FIRST, SECOND)            \
+    "v_alignbit_b32 %[a], " X0 ", " X0 ", %[r1]\n" BEFORE             \
     "v_xad_u32 " X3 ", " X3 ", %[m], " W "\n"                         \
-    "v_xor_b32_dpp %[c], %[a], %[a] quad_perm:[1,2,0,1]" SHA_ALL      \
-    "v_bitop3_b32 %[b], " X1 ", " X2 ", %[b] bitop3:0xe4\n" PARTNER   \
-    "v_xor_b32_dpp %[c], %[a], %[c] quad_perm:[2,0,1,2]" SHA_ALL      \
+    "v_bitop3_b32 %[b], " X0 ", " X1 ", %[m] bitop3:0xd2\n"           \
+    "v_xor_b32_dpp %[c], %[a], %[a] quad_perm:[1,2,0,1]" SHA_ALL FIRST \
+    "v_bitop3_b32 %[b], " X1 ", " X2 ", %[b] bitop3:0xe4\n"           \
+    "v_xor_b32_dpp %[c], %[a], %[c] quad_perm:[2,0,1,2]" SHA_ALL SECOND \
     "v_add3_u32 " X3 ", %[c], %[b], " X3 "\n"
-#define SHA_SLOT(S, X0, X1, X2, X3, W) S(X0, X1, X2, X3, W, "", SHA_PARTNER(X1, X3))
+#define SHA_SLOT(S, X0, X1, X2, X3, W) S(X0, X1, X2, X3, W, "", SHA_PARTNER(X1, X3), "")
 #define SHA_SLOT_TURN(S, X0, X1, X2, X3, W, FW, UNFED)                \
     S(X0, X1, X2, X3, W, "v_add_u32_e64 %[t], " FW ", " X1 "\n",      \
-      "v_add_u32_dpp " X3 ", %[t], " X3 " row_half_mirror" SHA_ON_E   \
+      "v_add_u32_dpp " X3 ", %[t], " X3 " row_half_mirror" SHA_ON_E,  \
       "v_add_u32_dpp " X3 ", " UNFED ", " X3 " row_half_mirror" SHA_ON_A)
 #define SHA_WORD(I) "v[%[words]+" I "]"
 #define SHA_FOUR(S, W0, W1, W2, W3)                                   \
@@ -1793,8 +1797,8 @@ __device__ __forceinline__ void sha_block_turn(ShaLanes& l, uint32_t word0, uint
     "v_mov_b32_e32 %[e2], %[x2]\nv_mov_b32_e32 %[e3], %[x3]\n"        \
     SHA_SLOT_TURN(S, "%[x0]", "%[x1]", "%[x2]", "%[x3]", W0, "%[f3]", "%[u1]") \
     SHA_SLOT_TURN(S, "%[x3]", "%[x0]", "%[x1]", "%[x2]", W1, "%[f2]", "%[u0]") \
-    SHA_FEED(SHA_ON_A, "%[f0]", "%[x2]") SHA_FEED(SHA_ON_A, "%[f1]", "%[x3]") \
-    SHA_FEED(SHA_ON_A, "%[f2]", "%[x0]") SHA_FEED(SHA_ON_A, "%[f3]", "%[x1]") \
+    SHA_FEED(SHA_ON_A, "%[f1]", "%[x3]") SHA_FEED(SHA_ON_A, "%[f2]", "%[x0]") \
+    SHA_FEED(SHA_ON_A, "%[f3]", "%[x1]") SHA_FEED(SHA_ON_A, "%[f0]", "%[x2]") \
     "v_mov_b32_e32 %[f0], %[x2]\nv_mov_b32_e32 %[f1], %[x3]\n"        \
     "v_mov_b32_e32 %[f2], %[x0]\nv_mov_b32_e32 %[f3], %[x1]\n"        \
     SHA_SLOT(S, "%[x2]", "%[x3]", "%[x0]", "%[x1]", W2)               \
