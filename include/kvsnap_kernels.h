@@ -153,8 +153,9 @@ int kvsnap_hash_records(const uint64_t* records, uint64_t record_bytes, int64_t 
                         uint32_t* crcs, int threads);
 
 /* At most 128 blocks between the cache and their records in one launch with no
- * device table before it: `records` (addresses of packed records, pinned or
- * device memory) and `blocks` are host arrays, read before the call returns.
+ * device table before it: `records` (8-byte aligned addresses of packed records,
+ * pinned or device memory) and `blocks` are host arrays, read before the call
+ * returns.
  * save != 0 writes the records, else the cache blocks.  tokens > 0 (a block's
  * token slots, the outermost axis of every span): a save's last record keeps
  * the first `filled` slots of each span, whose length / tokens is a multiple of

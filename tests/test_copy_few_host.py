@@ -144,3 +144,28 @@ def test_closed_sources_and_outside_targets_are_refused_before_the_launch(kernel
         with pytest.raises(RuntimeError):
             call()
     assert not any(name.startswith(("few", "gather", "restore")) for name, _ in kernels.launches)
+
+
+@pytest.mark.parametrize("save, mode", [(True, "staged"), (True, "direct"), (False, "dma"), (False, "kernel")])
+@pytest.mark.parametrize("shift", [0, 8, 1, 4])
+def test_records_off_the_word_boundaries_go_the_general_way(save, mode, shift):
+    """A reservation behind one of an odd size starts off an 8-byte boundary."""
+    found = FewKernels()
+    with patch.multiple(dataplane, kernel_library=lambda library=None: found, **CUDA_CHECKS):
+        held = caches("token", 9)
+        plane = plane_over(held, 4, **({"save_mode": mode} if save else {"restore_mode": mode,
+                                                                           "device_staging_bytes": 0}))
+        plane._place_stream = lambda: None
+        size = plane.block_bytes
+        slab = plane.pool.reserve(2 * size + shift)
+        assert slab.pointer % 16 == 0
+        targets = [(slab, shift), (slab, shift + size)]
+        if save:
+            plane.save_gather([2, 7], targets, 7)
+            assert slab.at(shift, size) == records_of(plane, [2], 4)[1]
+        else:
+            slab.fill(shift, records_of(plane, [2, 7], 8)[1])
+            found.launches.clear()
+            plane.load_scatter([4, 1], targets)
+            assert all(torch.equal(bits[[4, 1]], bits[[2, 7]]) for bits in cache_bits(held).values())
+    assert any(name.startswith("few") for name, _ in found.launches[:1]) == (shift % 8 == 0)

@@ -5,7 +5,8 @@ import ctypes as C
 import pytest
 import torch
 
-from kvsnap_amd.dataplane import _check, kernel_library
+from kvsnap_amd import synth
+from kvsnap_amd.dataplane import TorchBlockDataPlane, _check, kernel_library
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +66,23 @@ def test_bad_counts_are_refused(hip_library):
     one, ids = (C.c_uint64 * 129)(), (C.c_int64 * 129)()
     for n, spans, filled, tokens in ((129, 1, 0, 0), (-1, 1, 0, 0), (1, 1, 5, 4), (1, 1, 1, 0), (1, -1, 0, 0)):
         assert lib.kvsnap_copy_few(1, one, ids, n, t, t, t, t, spans, 8, filled, tokens, 12, 0) == -1
+
+
+def test_records_behind_an_odd_sized_reservation_round_trip(hip_library):
+    """Off the kernels' 8-byte boundaries a staged save and a copy-engine restore go the general way."""
+    caches, backing = synth.make_caches(4, 20, layout="vllm")
+    plane = TorchBlockDataPlane(caches, 16, 4 << 20, save_mode="staged", restore_mode="dma")
+    try:
+        odd = plane.pool.reserve(3)
+        staged, size = plane.pool.reserve(2 * plane.block_bytes), plane.block_bytes
+        assert staged.pointer % 8
+        targets = [(staged, 0), (staged, size)]
+        plane.save_gather([3, 9], targets, 32)
+        plane.load_scatter([12, 1], targets)
+        for tensor in caches.values():
+            bits = tensor.view(torch.int16)
+            assert torch.equal(bits[[12, 1]], bits[[3, 9]])
+        staged.close()
+        odd.close()
+    finally:
+        plane.close()
