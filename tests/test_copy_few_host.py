@@ -169,3 +169,35 @@ def test_records_off_the_word_boundaries_go_the_general_way(save, mode, shift):
             plane.load_scatter([4, 1], targets)
             assert all(torch.equal(bits[[4, 1]], bits[[2, 7]]) for bits in cache_bits(held).values())
     assert any(name.startswith("few") for name, _ in found.launches[:1]) == (shift % 8 == 0)
+
+
+@pytest.mark.parametrize("save", [True, False])
+def test_the_launch_is_made_with_the_plane_s_device_current(save, monkeypatch):
+    """The calling thread may have another device current."""
+    found, current, seen = FewKernels(), [], []
+    real = found.kvsnap_copy_few
+
+    class Current:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            current.append(self.device)
+
+        def __exit__(self, *exc):
+            current.pop()
+
+    def launch(*arguments):
+        seen.append(list(current))
+        return real(*arguments)
+
+    monkeypatch.setattr(found, "kvsnap_copy_few", launch)
+    with patch.multiple(dataplane, kernel_library=lambda library=None: found, **CUDA_CHECKS):
+        plane = plane_over(caches("token", 9), 4)
+        plane.torch.cuda.device = Current
+        targets = slabs(plane, 2, shared=True)
+        if save:
+            plane.save_gather([2, 7], targets, 8)
+        else:
+            plane.load_scatter([2, 7], targets)
+    assert seen == [[0]]

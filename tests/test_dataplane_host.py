@@ -175,7 +175,8 @@ class CpuCuda:
             return True
 
     def __init__(self):
-        self.cuda = SimpleNamespace(stream=lambda stream: nullcontext(), Event=self.Event,
+        self.cuda = SimpleNamespace(stream=lambda stream: nullcontext(), device=lambda index: nullcontext(),
+                                    Event=self.Event,
                                     current_stream=lambda device=None: MagicMock(cuda_stream=0),
                                     ExternalStream=lambda handle, device=None: MagicMock(cuda_stream=handle))
 
