@@ -144,10 +144,11 @@ int kvsnap_scatter_blocks(const void* records, int64_t record_pitch, const int64
 
 /* SHA-256 (32 bytes each) and CRC32C of n records of record_bytes in host
  * memory, on at most `threads` host threads (1 to 256; the caller's is one of
- * them, the others end before the call does).  Needs a CPU with the SHA and
- * SSE4.2 instructions: kvsnap_hash_records_available() is 1 there, else 0.  No
- * GPU call is made.  (The reference hashes on host threads,
- * kvsnap/connector/volatile.py:151.) */
+ * them, the others end before the call does, and calls at the same time share
+ * them: none starts one while threads - 1 others help calls of this process).
+ * Needs a CPU with the SHA and SSE4.2 instructions:
+ * kvsnap_hash_records_available() is 1 there, else 0.  No GPU call is made.
+ * (The reference hashes on host threads, kvsnap/connector/volatile.py:151.) */
 int kvsnap_hash_records_available(void);
 int kvsnap_hash_records(const uint64_t* records, uint64_t record_bytes, int64_t n_records, uint8_t* digests,
                         uint32_t* crcs, int threads);

@@ -5,7 +5,9 @@
 // issue time (0.97 us a 64-byte block) however few records there are, while a
 // host core with the SHA extensions runs a chain some 35 times as fast.  A save
 // of few records hashes sooner here, from the pinned records it has just
-// written; many records hash sooner on the GPU, beside their copies.
+// written; many records hash sooner on the GPU, beside their copies.  Callers
+// share the helping threads: all of a process's calls together start no more
+// than one of them asked for.
 #include "common.h"
 
 #include <algorithm>
@@ -137,9 +139,23 @@ KVSNAP_SHA_TARGET void hash_lanes(const uint8_t* const* records, uint64_t nbytes
     }
 }
 
+std::atomic<int> g_helpers{0};  // threads of this process that help a call now
+
+bool take_helper(int most) {
+    int now = g_helpers.load(std::memory_order_relaxed);
+    while (now < most)
+        if (g_helpers.compare_exchange_weak(now, now + 1, std::memory_order_relaxed)) return true;
+    return false;
+}
+
 void hash_records(const uint64_t* records, uint64_t nbytes, int64_t n, uint8_t* digests, uint32_t* crcs, int threads) {
-    // Pairs of records once every thread has one; a thread takes the next when it is done with its last.
-    const int64_t lanes = n > threads ? 2 : 1, jobs = (n + lanes - 1) / lanes;
+    // A thread is worth starting (about 15 us) for 64 KiB of its own, and has one record or, where there are more
+    // records than threads, pairs of them; it takes the next when it is done with its last.
+    const int64_t pairs = (n + 1) / 2;
+    const int64_t useful = std::min<int64_t>({threads, n > threads ? pairs : n, static_cast<int64_t>(nbytes * n >> 16)});
+    int64_t helpers = 0;
+    while (helpers + 1 < useful && take_helper(threads - 1)) ++helpers;
+    const int64_t lanes = n > helpers + 1 ? 2 : 1, jobs = (n + lanes - 1) / lanes;
     std::atomic<int64_t> next{0};
     const auto work = [&] {
         for (int64_t job; (job = next.fetch_add(1, std::memory_order_relaxed)) < jobs;) {
@@ -160,13 +176,17 @@ void hash_records(const uint64_t* records, uint64_t nbytes, int64_t n, uint8_t* 
         }
     };
     std::vector<std::thread> others;
-    // A thread is worth starting (about 15 us) for 64 KiB of its own.
-    const int64_t useful = std::min<int64_t>({threads, jobs, static_cast<int64_t>(nbytes * n >> 16)});
-    others.reserve(static_cast<size_t>(std::max<int64_t>(useful, 1)));
+    int64_t untaken = helpers;
     try {
-        for (int64_t i = 1; i < useful; ++i) others.emplace_back(work);
+        others.reserve(static_cast<size_t>(helpers));
+        for (; untaken > 0; --untaken)
+            others.emplace_back([&work] {
+                work();
+                g_helpers.fetch_sub(1, std::memory_order_relaxed);
+            });
     } catch (...) {
         // No more threads to be had: the ones there are, this one at least, do all the work.
+        g_helpers.fetch_sub(static_cast<int>(untaken), std::memory_order_relaxed);
     }
     work();
     for (auto& thread : others) thread.join();
