@@ -1,9 +1,10 @@
-"""Records hashed on host threads: the native function against hashlib and the oracle, and which saves take it."""
+"""Records hashed on host threads: the native function against hashlib and the oracle, which saves take it, and what
+waits for it (not the save)."""
 import ctypes as C
 import hashlib
 import os
 import threading
-from unittest.mock import patch
+from unittest.mock import MagicMock, patch
 
 import numpy as np
 import pytest
@@ -11,8 +12,12 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from kvsnap_amd import dataplane, native
+from kvsnap_amd.blobs import BlobDirectory
+from kvsnap_amd.host_tier import HostTier
+from kvsnap_amd.pool import CopyFailed, CudaPool
 from tests.test_copy_few_host import CUDA_CHECKS, FewKernels, caches
-from tests.test_dataplane_host import plane_over, slabs
+from tests.test_dataplane_host import CpuCuda, plane_over, slabs
+from tests.test_pool import fake_pool_path      # noqa: F401 (a fixture)
 
 LIBRARY = native.kernel_library()
 needs_sha = pytest.mark.skipif(not LIBRARY.kvsnap_hash_records_available(), reason="no SHA instructions here")
@@ -95,9 +100,9 @@ def kernels(monkeypatch):
 @pytest.mark.parametrize("shared", [True, False], ids=["one-allocation", "allocation-each"])
 @pytest.mark.parametrize("chunk", [1, 3, 1 << 20])
 @pytest.mark.parametrize("tokens", [1, 39, 44])
-def test_a_save_of_few_records_has_their_digests_when_it_returns(kernels, oracle_lib, monkeypatch, few_bytes, mode,
-                                                                 shared, tokens, chunk):
+def test_the_digests_of_a_save_of_few_records(kernels, oracle_lib, monkeypatch, few_bytes, mode, shared, tokens, chunk):
     monkeypatch.setattr(dataplane, "FEW_BYTES", few_bytes)
+    monkeypatch.setattr(CpuCuda.Event, "query", lambda self: False)     # parts that have landed are taken together
     plane = plane_over(caches("token", 14), 4, save_mode=mode)
     ids = [7, 2, 5, 0, 8, 13, 1, 9, 4, 11, 3][:-(-tokens // 4)]
     targets, plain, digests = slabs(plane, len(ids), shared=shared), slabs(plane, len(ids), shared=shared), []
@@ -107,27 +112,150 @@ def test_a_save_of_few_records_has_their_digests_when_it_returns(kernels, oracle
     assert count == (-(-len(ids) // chunk) if mode == "direct" else 1 if shared else len(ids))
     records = [a.at(offset, plane.block_bytes) for a, offset in targets]
     assert records == [a.at(offset, plane.block_bytes) for a, offset in plain]
-    assert len(digests) == 1 and digests[0].ready()
+    assert len(digests) == 1
     assert digests[0].result() == [(hashlib.sha256(r).hexdigest(), oracle_lib.crc32c(np.frombuffer(r, np.uint8)))
                                    for r in records]
     assert sum(kernels.parts) == len(ids) and max(kernels.parts) <= (4 if not few_bytes else len(ids))
 
 
+def expected(records):
+    import oracle
+    return [(hashlib.sha256(r).hexdigest(), oracle.crc32c(r)) for r in records]
+
+
+class Held:
+    """A plane on the library's own pool whose host hashes wait for ``open``."""
+
+    def __init__(self, kernels, pool_path, mode):
+        self.open, self.begun, self.fail = threading.Event(), threading.Event(), False
+        real = kernels.kvsnap_hash_records
+
+        def hashing(*arguments):
+            self.begun.set()
+            assert self.open.wait(5)
+            return -1 if self.fail else real(*arguments)
+
+        kernels.kvsnap_hash_records = hashing
+        self.plane = plane_over(caches("token", 14), 4, save_mode=mode)
+        self.size = self.plane.block_bytes
+        self.plane.pool = CudaPool(12 * self.size, 0, library=pool_path)
+
+    def save(self, ids=(3, 1, 4, 11, 5, 9)):
+        staged, digests = self.plane.pool.reserve(len(ids) * self.size), []
+        targets = [(staged, i * self.size) for i in range(len(ids))]
+        self.plane.save_gather(list(ids), targets, 4 * len(ids), digests=digests)
+        return staged, targets, digests[0], [C.string_at(staged.pointer + at, self.size) for _, at in targets]
+
+
+@pytest.fixture(params=[("staged", 0), ("staged", 1 << 20), ("direct", 0)], ids=["parts", "one-launch", "direct"])
+def held(request, kernels, monkeypatch, fake_pool_path):       # noqa: F811
+    monkeypatch.setattr(dataplane, "FEW_BYTES", request.param[1])
+    found = Held(kernels, fake_pool_path, request.param[0])
+    yield found
+    found.open.set()
+    found.plane.close()
+
+
+def after(held, call):
+    """``call`` in a thread of its own: it must wait until the hashes go on."""
+    thread = threading.Thread(target=call)
+    thread.start()
+    thread.join(0.2)
+    assert thread.is_alive()
+    held.open.set()
+    thread.join(20)
+    assert not thread.is_alive()
+
+
 @needs_sha
-def test_a_target_closed_meanwhile_fails_the_save_and_gives_no_digests(kernels, monkeypatch):
-    monkeypatch.setattr(dataplane, "FEW_BYTES", 0)
-    plane = plane_over(caches("token", 14), 4)
-    targets, digests = slabs(plane, 9, shared=False), []
-    real = kernels.kvsnap_hash_records
+def test_a_save_returns_when_its_records_have_landed(held):
+    staged, _, digests, records = held.save()
+    assert held.begun.wait(5) and not digests.ready() and staged.ready()
+    staged.wait()                                            # its copies; the pool is free meanwhile
+    held.plane.pool.reserve(held.size).close()
+    after(held, digests.result)
+    assert digests.ready() and digests.result() == expected(records)
 
-    def closing(*arguments):
-        targets[5][0].closed = True
-        return real(*arguments)
 
-    kernels.kvsnap_hash_records = closing
-    with pytest.raises(RuntimeError):
-        plane.save_gather(list(range(9)), targets, 36, digests=digests)
-    assert not digests and kernels.parts == [4]
+@needs_sha
+def test_closing_a_target_waits_until_its_records_are_read(held):
+    staged, _, digests, records = held.save()
+    assert held.begun.wait(5)
+    after(held, staged.close)
+    assert staged.closed and digests.result() == expected(records)
+
+
+@needs_sha
+@pytest.mark.parametrize("write", ["save", "write", "zero", "copy"])
+def test_writing_a_target_waits_until_its_records_are_read(held, write):
+    staged, targets, digests, records = held.save()
+    other = held.plane.pool.reserve(held.size)
+    assert held.begun.wait(5)
+    buffer = C.create_string_buffer(held.size)
+    # Elsewhere nothing waits.
+    held.plane.save_gather([2], [(other, 0)], 4)
+    after(held, {"save": lambda: held.plane.save_gather([2], targets[3:4], 4),
+                 "write": lambda: staged.write(bytes(6 * held.size)),
+                 "zero": lambda: staged.zero(held.size + 3, 5),
+                 "copy": lambda: staged.copy(C.addressof(buffer), held.size, held.size, to_host=True)}[write])
+    staged.wait()
+    assert digests.result() == expected(records)
+    assert [C.string_at(staged.pointer + at, held.size) for _, at in targets] != records
+
+
+@needs_sha
+def test_a_hash_that_fails_is_raised_by_result(held):
+    held.fail = True
+    held.open.set()
+    staged, _, digests, _ = held.save()
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            digests.result()
+    staged.close()
+
+
+@needs_sha
+def test_a_plane_closed_meanwhile_finishes_its_hashes(held):
+    staged, _, digests, records = held.save()
+    assert held.begun.wait(5)
+    after(held, held.plane.close)
+    assert staged.closed and digests.result() == expected(records)
+
+
+@needs_sha
+def test_without_a_thread_result_does_the_work(held, monkeypatch):
+    monkeypatch.setattr(dataplane, "HostHashes", MagicMock(side_effect=RuntimeError("can't start new thread")))
+    held.open.set()
+    staged, _, digests, records = held.save()
+    assert digests.result() == expected(records)
+
+
+@needs_sha
+@pytest.mark.parametrize("tier", ["host", "blobs"])
+@pytest.mark.parametrize("fail", [False, True])
+def test_the_blocks_are_free_before_the_hashes(held, tmp_path, tier, fail):
+    """``fenced`` is set when the records have landed; a hash that fails is not an unproven copy."""
+    fenced, found = threading.Event(), []
+    held.fail = fail
+
+    def save():
+        try:
+            if tier == "host":
+                found.append(HostTier(held.plane, 1 << 20).save([3, 1, 4], 12, fenced=fenced))
+            else:
+                found.append(BlobDirectory(tmp_path).save(held.plane, [3, 1, 4], 12, fenced=fenced))
+        except Exception as exc:
+            found.append(exc)
+
+    saver = threading.Thread(target=save)
+    saver.start()
+    assert held.begun.wait(5) and fenced.wait(2) and saver.is_alive()
+    held.open.set()
+    saver.join(20)
+    if fail:
+        assert type(found[0]) is RuntimeError and not isinstance(found[0], CopyFailed)
+    else:
+        assert [len(segment["blob_id"]) for segment in found[0]["segments"]] == [64] * 3
 
 
 def test_the_rule(kernels, monkeypatch):
