@@ -115,7 +115,19 @@ def test_the_digests_of_a_save_of_few_records(kernels, oracle_lib, monkeypatch, 
     assert len(digests) == 1
     assert digests[0].result() == [(hashlib.sha256(r).hexdigest(), oracle_lib.crc32c(np.frombuffer(r, np.uint8)))
                                    for r in records]
-    assert sum(kernels.parts) == len(ids) and max(kernels.parts) <= (4 if not few_bytes else len(ids))
+    if few_bytes and chunk >= len(ids):
+        assert kernels.parts == [len(ids)]
+    else:
+        assert kernels.parts == [b - a for low in range(0, len(ids), chunk)
+                                 for a, b in dataplane._parts(low, min(low + chunk, len(ids)), 4)]
+
+
+def test_parts():
+    """Each twice the one before, and a last one that takes a rest of less than half of it along."""
+    sizes = lambda n, part: [b - a for a, b in dataplane._parts(0, n, part)]
+    assert sizes(128, 16) == [16, 32, 80] and sizes(64, 16) == [16, 32, 16] and sizes(32, 16) == [16, 16]
+    assert sizes(23, 16) == [23] and sizes(24, 16) == [16, 8] and sizes(1, 16) == [1] and sizes(0, 16) == []
+    assert sizes(7, 1) == [1, 2, 4] and dataplane._parts(5, 12, 4) == [(5, 9), (9, 12)]
 
 
 def expected(records):
