@@ -46,8 +46,33 @@ def oracle_lib():
     return oracle
 
 
+@pytest.fixture(params=["general", "few-blocks"])
+def copy_routes(request, monkeypatch):
+    """Both routes of a small save or restore: the general one, which large ones take too (device staging, copy
+    engines, launch tables, hashes on the GPU), and the one it takes by itself (one launch for few blocks, few
+    records hashed on the host)."""
+    from kvsnap_amd import dataplane
+    if request.param == "general":
+        monkeypatch.setattr(dataplane, "FEW_BLOCKS", 0)
+        monkeypatch.setattr(dataplane, "HASH_THREADS", 0)
+    return request.param
+
+
 @pytest.fixture
-def planes(hip_library):
+def hashed_as(copy_routes):
+    """Asserts that a save of ``n`` records was hashed where its route says, and returns its job."""
+    from kvsnap_amd import dataplane
+
+    def check(digests, plane, n):
+        on_host = copy_routes != "general" and plane._hash_threads(dataplane.kernel_library(), n)
+        assert type(digests._event) is (dataplane.HostHashJob if on_host else dataplane.HashJob)
+        return digests._event
+
+    return check
+
+
+@pytest.fixture
+def planes(hip_library, copy_routes):
     """A maker of warmed-up data planes (block size 16 unless asked), each closed when the test ends."""
     import torch
     from kvsnap_amd.dataplane import TorchBlockDataPlane

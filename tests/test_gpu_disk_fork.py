@@ -23,7 +23,7 @@ from kvsnap_amd import synth
 from kvsnap_amd.blobs import HEADER, BlobDirectory
 from kvsnap_amd.dataplane import TorchBlockDataPlane
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("copy_routes")]
 
 LAYERS, BLOCKS, BLOCK_SIZE = 36, 640, 16
 SESSION, SHARED = 160, 120          # blocks of each session; the child's first SHARED copy the parent's

@@ -19,7 +19,7 @@ from kvsnap_amd.blobs import CorruptSnapshotError
 from kvsnap_amd.dataplane import TorchBlockDataPlane
 from kvsnap_amd.host_tier import HostTier
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("copy_routes")]
 
 LAYERS, BLOCKS, BLOCK_SIZE = 4, 64, 16
 

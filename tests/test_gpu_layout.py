@@ -23,7 +23,7 @@ from kvsnap_amd.host_tier import HostTier
 from kvsnap_amd.layout import LayoutMismatch
 from kvsnap_amd.worker import KvsnapMetadata, KvsnapWorker, Transfer
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("copy_routes")]
 
 LAYERS, BLOCKS, BLOCK_SIZE, SESSION = 4, 64, 16, 12
 

@@ -167,7 +167,8 @@ def test_the_split_restore_and_hash_streams_are_the_plane_s_own_and_distinct(pla
     assert set(others) <= set(plane._owned_streams)
 
 
-def test_a_plane_closed_with_work_in_flight_and_an_exception_alive_exits_cleanly(hip_library, tmp_path):
+@pytest.mark.parametrize("hash_threads", ["0", "8"])
+def test_a_plane_closed_with_work_in_flight_and_an_exception_alive_exits_cleanly(hip_library, tmp_path, hash_threads):
     """A test process once crashed at exit after a failing test: pinned tensors copied ``non_blocking`` on the
     plane's own streams, kept alive by the failure's traceback, were freed after ``close`` had destroyed
     those streams, and torch's pinned allocator then queried events recorded on them.  The plane no longer
@@ -208,7 +209,8 @@ for _ in range(4):                     # the pinned allocator processes its even
 torch.cuda.synchronize()
 print("clean exit", flush=True)
 """)
-    env = dict(__import__("os").environ, PYTHONPATH=str(__import__("pathlib").Path(__file__).resolve().parents[1]))
+    env = dict(__import__("os").environ, PYTHONPATH=str(__import__("pathlib").Path(__file__).resolve().parents[1]),
+               KVSNAP_HASH_THREADS=hash_threads)
     done = subprocess.run([sys.executable, str(script)], capture_output=True, text=True, timeout=120, env=env)
     assert done.returncode == 0 and "clean exit" in done.stdout, (done.returncode, done.stdout[-2000:],
                                                                   done.stderr[-2000:])
@@ -256,7 +258,7 @@ def test_save_gather_matches_the_oracle_records_and_zeroes_the_tail(planes, orac
             allocation.close()
 
 
-def test_gpu_digests_match_the_oracle_and_hashlib(planes, oracle_lib):
+def test_gpu_digests_match_the_oracle_and_hashlib(planes, oracle_lib, hashed_as):
     caches, backing = synth.make_caches(LAYERS, 40, layout="vllm")
     plane = planes(caches)
     keep = synth.fill(plane, 9)
@@ -269,6 +271,7 @@ def test_gpu_digests_match_the_oracle_and_hashlib(planes, oracle_lib):
     targets = [(staged, i * size) for i in range(len(block_ids))]
     digests = []
     plane.save_gather(block_ids, targets, tokens, digests=digests)
+    hashed_as(digests[0], plane, 17)
     got = digests[0].result()
     for index, (hexdigest, crc) in enumerate(got):
         record = C.string_at(staged.pointer + index * size, size)
@@ -279,7 +282,8 @@ def test_gpu_digests_match_the_oracle_and_hashlib(planes, oracle_lib):
 
 @pytest.mark.parametrize("lead", [True, False], ids=["lead-stream", "one-gather"])
 @pytest.mark.parametrize("layout", ["vllm", "kv_split"])
-def test_a_hashed_save_gathered_over_two_streams_matches_the_oracle(planes, oracle_lib, monkeypatch, layout, lead):
+def test_a_hashed_save_gathered_over_two_streams_matches_the_oracle(planes, oracle_lib, monkeypatch, hashed_as,
+                                                                    layout, lead):
     """A hashed save longer than one chunk: its first chunk is gathered on the copy stream and the rest,
     with the last record's tail, on the lead stream, whose copies wait for it.  Records, CRC32C and SHA-256
     equal the oracle's with the lead stream and without it."""
@@ -304,6 +308,7 @@ def test_a_hashed_save_gathered_over_two_streams_matches_the_oracle(planes, orac
                    else [(allocation, 0) for allocation in owned])
         digests = []
         assert plane.save_gather(block_ids, targets, tokens, chunk_bytes=2 * size, digests=digests) == copies
+        hashed_as(digests[0], plane, 7)
         for index, (allocation, offset) in enumerate(targets):
             assert np.array_equal(pinned_bytes(allocation, offset, size), records[index]), (kind, index)
         for index, ((hexdigest, crc), record) in enumerate(zip(digests[0].result(), records)):
@@ -477,7 +482,7 @@ def test_sha256_ranges_of_several_record_sets_in_one_launch_equal_hashlib(hip_li
         _check(lib, lib.kvsnap_sha256_ranges(9, one[0], one[1], one[2], n_one, one[3], one[4], one[5], one[6], stream))
 
 
-def test_saves_that_share_one_hash_stream_hash_side_by_side_and_equal_the_oracle(oracle_lib, monkeypatch):
+def test_saves_that_share_one_hash_stream_hash_side_by_side_and_equal_the_oracle(oracle_lib, monkeypatch, hashed_as):
     """With one hash stream, three saves issued from three threads share each SHA-256 launch (their chains
     advance together instead of one save after another); every save's ids and CRC32Cs equal the oracle's
     digests of its pinned records."""
@@ -513,6 +518,7 @@ def test_saves_that_share_one_hash_stream_hash_side_by_side_and_equal_the_oracle
         assert not errors, errors
         assert plane.stream_report()["hash_streams"] == 1
         for i, ids in enumerate(sessions):
+            hashed_as(found[i][0], plane, len(ids))
             crcs, shas = oracle_lib.digest_records(pinned[i].pointer, size, size, len(ids), threads=4)
             assert found[i][0].result() == [(bytes(h).hex(), int(c)) for h, c in zip(shas, crcs)], i
         for p in pinned:
@@ -610,7 +616,7 @@ def test_restore_from_device_memory_uses_the_same_kernel(planes):
 
 
 @pytest.mark.parametrize("layout", ["vllm", "kv_split"])
-def test_direct_save_writes_pinned_records_in_place(hip_library, oracle_lib, layout):
+def test_direct_save_writes_pinned_records_in_place(hip_library, oracle_lib, hashed_as, layout):
     caches, backing = synth.make_caches(LAYERS, 24, layout=layout)
     plane = TorchBlockDataPlane(caches, BLOCK_SIZE, 64 << 20, save_mode="direct")
     try:
@@ -629,6 +635,7 @@ def test_direct_save_writes_pinned_records_in_place(hip_library, oracle_lib, lay
                        else [(allocation, 0) for allocation in owned])
             digests = []
             assert plane.save_gather(block_ids, targets, tokens, chunk_bytes=2 * size, digests=digests) == 3
+            hashed_as(digests[0], plane, 5)
             for index, (allocation, offset) in enumerate(targets):
                 assert np.array_equal(pinned_bytes(allocation, offset, size), records[index]), (kind, index)
             for (hexdigest, crc), record in zip(digests[0].result(), records):
@@ -979,7 +986,8 @@ def test_the_gather_with_crc32c_follows_any_groups_table(oracle_lib, groups, n, 
 
 
 @pytest.mark.parametrize("tokens", [12 * BLOCK_SIZE, 12 * BLOCK_SIZE - 7])
-def test_a_hashed_direct_save_is_one_checked_gather_and_its_digests_are_the_oracle_s(planes, oracle_lib, tokens):
+def test_a_hashed_direct_save_is_one_checked_gather_and_its_digests_are_the_oracle_s(planes, oracle_lib, hashed_as,
+                                                                                     copy_routes, tokens):
     """save_mode="direct" with digests: the checked gather writes the pinned records and their device copy and
     folds their CRC32Cs in one pass over the cache; the SHA-256 reads the device copy.  Records (last tail zeroed),
     CRC32Cs and SHA-256s equal the oracle's."""
@@ -995,6 +1003,8 @@ def test_a_hashed_direct_save_is_one_checked_gather_and_its_digests_are_the_orac
     staged = plane.pool.reserve(12 * size)
     digests = []
     assert plane.save_gather(saved, [(staged, i * size) for i in range(12)], tokens, digests=digests) == 1
+    job = hashed_as(digests[0], plane, 12)
+    assert copy_routes != "general" or job.crc_given
     got = digests[0].result()
     if tokens % BLOCK_SIZE:
         oracle_lib.zero_tail(expected[11], plane.layers, tokens % BLOCK_SIZE)
@@ -1045,7 +1055,8 @@ def test_a_checked_restore_loads_clean_blocks_and_reports_a_corrupt_one_only_aft
 @pytest.mark.parametrize("heads", [1, 2, 4])
 @pytest.mark.parametrize("layout", ["kv_split", "vllm"])
 @pytest.mark.parametrize("restore_mode", ["kernel", "dma"])
-def test_a_tensor_parallel_shard_round_trips_with_short_spans(planes, oracle_lib, layout, restore_mode, heads):
+def test_a_tensor_parallel_shard_round_trips_with_short_spans(planes, oracle_lib, hashed_as, copy_routes, layout,
+                                                              restore_mode, heads):
     """One tensor-parallel rank's shard of Qwen3-8B (TP = 8, 4 and 2: 1, 2 and 4 KV heads, 4-16 KiB K/V spans,
     8-32 KiB vLLM spans), where the copy launches put several spans in one workgroup and a hashed save takes
     the gather with CRC32C: the gathered records equal the oracle's fill, their digests the oracle's, and the
@@ -1065,6 +1076,8 @@ def test_a_tensor_parallel_shard_round_trips_with_short_spans(planes, oracle_lib
     targets = [(staged, i * size) for i in range(128)]
     digests = []
     plane.save_gather(saved, targets, 128 * 16 - 5, digests=digests)
+    job = hashed_as(digests[0], plane, 128)
+    assert copy_routes != "general" or job.crc_given            # by the gather
     got = digests[0].result()
     crcs, shas = oracle_lib.digest_records(staged.pointer, size, size, 128, threads=16)
     assert [crc for _, crc in got] == crcs.tolist()

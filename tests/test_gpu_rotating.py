@@ -25,7 +25,7 @@ torch = pytest.importorskip("torch")
 from kvsnap_amd import synth
 from kvsnap_amd.dataplane import TorchBlockDataPlane, _check, kernel_library
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("copy_routes")]
 
 LAYERS, BLOCKS, BLOCK_SIZE = 28, 2048, 16
 SESSION_TOKENS = (1024, 2048, 4096, 8192)

@@ -18,7 +18,7 @@ from kvsnap_amd.dataplane import TorchBlockDataPlane
 from kvsnap_amd.host_tier import HostTier
 from kvsnap_amd.worker import KvsnapMetadata, KvsnapWorker, Transfer
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("copy_routes")]
 
 LAYERS, BLOCKS, BLOCK_SIZE = 4, 96, 16
 
