@@ -1,5 +1,6 @@
 """Which calls go through kvsnap_copy_few, and that each leaves what the general path leaves (CPU kernels)."""
 import ctypes as C
+from contextlib import nullcontext
 from unittest.mock import patch
 
 import pytest
@@ -106,7 +107,7 @@ def test_restores_equal_the_general_path(kernels, mode):
 
 
 def test_the_rule(monkeypatch):
-    """At most 128 blocks, one chunk, no timer; FEW_BYTES for staged saves and dma restores."""
+    """At most 128 blocks, one chunk; FEW_BYTES for staged saves and dma restores."""
     found = FewKernels()
     with patch.multiple(dataplane, kernel_library=lambda library=None: found, **CUDA_CHECKS):
         held = caches("token", 140)
@@ -116,7 +117,6 @@ def test_the_rule(monkeypatch):
             plane = plane_over(held, 4, **({"save_mode": mode} if save else {"restore_mode": mode,
                                                                                "device_staging_bytes": 0}))
             plane._place_stream = lambda: None
-            plane.timer = options.pop("timer", None)
             targets = slabs(plane, n, shared=True)
             found.launches.clear()
             if save:
@@ -201,3 +201,27 @@ def test_the_launch_is_made_with_the_plane_s_device_current(save, monkeypatch):
         else:
             plane.load_scatter([2, 7], targets)
     assert seen == [[0]]
+
+
+@pytest.mark.parametrize("save, name", [(True, "gather_to"), (False, "restore")])
+def test_a_timer_times_the_launch_and_does_not_change_it(save, name):
+    class Timer:
+        spans = []
+
+        def wants(self, wanted):
+            return True
+
+        def span(self, wanted, stream):
+            self.spans.append(wanted)
+            return nullcontext()
+
+    found = FewKernels()
+    with patch.multiple(dataplane, kernel_library=lambda library=None: found, **CUDA_CHECKS):
+        plane = plane_over(caches("token", 9), 4)
+        plane.timer = Timer()
+        targets = slabs(plane, 2, shared=True)
+        if save:
+            plane.save_gather([2, 7], targets, 8)
+        else:
+            plane.load_scatter([2, 7], targets)
+    assert found.launches == [("few_save" if save else "few_restore", 2)] and Timer.spans == [name]
