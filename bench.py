@@ -69,13 +69,11 @@ PCIE5_X16_GBPS = round(32 * 16 * 128 / 130 / 8, 2)
 # round wave issues 534 VALU per 64-byte block (the assembly of SHA_BLOCK: 64
 # slots of alignbit, 2 bitop3, xad, 3 DPP, add3, and 22 at the block's turn); a
 # wave64 VALU takes 4 cycles of its SIMD at the 2.4 GHz peak engine clock.  All
-# chains run side by side (one round wave per 8 records).  The two-lane form's
-# 9-VALU slot is also timed live on one wave (kvsnap_sha_round_probe: shader
-# cycles and the 100 MHz constant clock), which gives the rate instructions
-# issue at and the engine clock meanwhile; the bound at that rate (8 of its 9
-# instructions a slot) is reported beside the nominal one.
+# chains run side by side (one round wave per 8 records).  The form's 8-VALU
+# slot is also timed live on one wave (kvsnap_sha_round_probe: shader cycles and
+# the 100 MHz constant clock), which gives the rate a slot runs at and the engine
+# clock meanwhile; the bound at that rate is reported beside the nominal one.
 SHA_VALU_PER_BLOCK = 534
-SHA_SLOT_VALU, SHA_PROBE_SLOT_VALU = 8, 9
 SHA_CYCLES_PER_VALU = 4
 ENGINE_CLOCK_GHZ = 2.4
 SHA_PROBE_SLOTS = 1 << 18
@@ -119,7 +117,7 @@ def sha_issue_bound(record_bytes, records, ms, round_rate):
     bound_ms = blocks * SHA_VALU_PER_BLOCK * SHA_CYCLES_PER_VALU / (ENGINE_CLOCK_GHZ * 1e6)
     total = record_bytes * records
     slot_cycles, clock_ghz = round_rate
-    sequence_ms = blocks * 64 * slot_cycles * SHA_SLOT_VALU / SHA_PROBE_SLOT_VALU / (ENGINE_CLOCK_GHZ * 1e6)
+    sequence_ms = blocks * 64 * slot_cycles / (ENGINE_CLOCK_GHZ * 1e6)
     fips_ms = blocks * (64 * SHA_FIPS_TWO_LANE_ROUND + SHA_FIPS_FEED_FORWARD) * SHA_CYCLES_PER_VALU / (
         ENGINE_CLOCK_GHZ * 1e6)
     one_lane_ms = blocks * (64 * SHA_FIPS_ROUND_INSTRUCTIONS + 2 * SHA_FIPS_FEED_FORWARD) * SHA_CYCLES_PER_VALU / (
@@ -134,7 +132,7 @@ def sha_issue_bound(record_bytes, records, ms, round_rate):
             "achieved": round(total / (ms * 1e6), 2), "peak": round(total / (bound_ms * 1e6), 2), "unit": "GB/s",
             "frac": round(bound_ms / ms, 4), "round_cycles_measured": round(slot_cycles, 2),
             "round_probe_clock_ghz": round(clock_ghz, 3),
-            "round_probe": "kvsnap_sha_round_probe: the two-lane round sequence (9 VALU) alone on one wave, "
+            "round_probe": "kvsnap_sha_round_probe: the quad form's round sequence (8 VALU) alone on one wave, "
                            "s_memtime / s_memrealtime",
             "round_sequence_bound_ms": round(sequence_ms, 3), "frac_of_round_sequence_rate": round(sequence_ms / ms, 4)}
 

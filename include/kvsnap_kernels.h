@@ -245,7 +245,7 @@ int kvsnap_sha256_ranges(int count, const uint64_t* records, const uint64_t* rec
                          const uint64_t* end_blocks, const uint64_t* states, const uint64_t* outs, uintptr_t stream);
 
 /* The SHA-256 round's own issue rate, measured on the GPU: one wave runs
- * `reps` (a multiple of 16) slots of the two-lane form's round sequence with no
+ * `reps` (a multiple of 16) slots of the quad form's round sequence with no
  * memory traffic, and out (3 device words) receives the shader-clock cycles,
  * the 100 MHz constant-clock ticks and a checksum.  No reference
  * counterpart: the bench's SHA-256 bound is priced from it. */

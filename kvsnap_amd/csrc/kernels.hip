@@ -2141,8 +2141,8 @@ __global__ __launch_bounds__(kShaThreads) void sha256_ranges_kernel(ShaRanges ra
                                  blockIdx.x);
 }
 
-// The round's own issue rate, measured: one wave runs `reps` slots of the
-// two-lane form's instruction sequence (SHA_TWO, both halves) on values seeded
+// The round's own issue rate, measured: one wave runs `reps` slots of the quad
+// form's instruction sequence (SHA_QUAD, both halves) on values seeded
 // per lane, with no LDS, no waits and no barrier, between two reads of the
 // shader clock (s_memtime) and of the 100 MHz constant clock (s_memrealtime).
 // out[0] = shader cycles, out[1] = constant-clock ticks, out[2] = a checksum
@@ -2152,7 +2152,7 @@ constexpr int kShaProbeUnroll = 16;
 __global__ __launch_bounds__(64) void sha_round_probe_kernel(uint32_t seed, int reps, uint64_t* __restrict__ out) {
     const int lane = threadIdx.x;
     const bool a_lane = (lane >> 2) & 1;
-    ShaHalf half = ShaTwoLane::lanes(a_lane, lane);
+    ShaQuarter half = ShaQuad::lanes(a_lane, lane);
     opaque(half.m);
     uint32_t x[4];
 #pragma unroll
@@ -2165,11 +2165,11 @@ __global__ __launch_bounds__(64) void sha_round_probe_kernel(uint32_t seed, int 
     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
     for (int r = 0; r < rounds; ++r) {
         uint32_t a, b, c;
-#define SHA_PROBE_FOUR SHA_FOUR(SHA_TWO, "%[w]", "%[w]", "%[w]", "%[w]")
+#define SHA_PROBE_FOUR SHA_FOUR(SHA_QUAD, "%[w]", "%[w]", "%[w]", "%[w]")
         asm volatile(".p2align 3\n" SHA_PROBE_FOUR SHA_PROBE_FOUR SHA_PROBE_FOUR SHA_PROBE_FOUR
                      : [x0] "+v"(x[0]), [x1] "+v"(x[1]), [x2] "+v"(x[2]), [x3] "+v"(x[3]), [a] "=&v"(a),
                        [b] "=&v"(b), [c] "=&v"(c)
-                     : [r1] "v"(half.r1), [r2] "v"(half.r2), [r3] "v"(half.r3), [m] "v"(half.m), [w] "v"(word));
+                     : [r1] "v"(half.r), [m] "v"(half.m), [w] "v"(word));
 #undef SHA_PROBE_FOUR
     }
     const uint64_t c1 = __builtin_amdgcn_s_memtime();

@@ -1310,7 +1310,7 @@ def test_pipelined_disk_restore_is_byte_exact_and_refuses_corrupt_blobs(planes, 
 
 
 def test_the_sha_round_probe_times_the_round_sequence(hip_library):
-    """kvsnap_sha_round_probe: the round sequence on one wave takes at least its 9 VALU at 4 cycles each a slot
+    """kvsnap_sha_round_probe: the round sequence on one wave takes at least its 8 VALU at 4 cycles each a slot
     (and not wildly more), the engine clock it reports is a plausible MI355X clock, and the slots were run (the
     checksum depends on the seed)."""
     out = torch.zeros(3, dtype=torch.int64, device="cuda")
@@ -1323,7 +1323,7 @@ def test_the_sha_round_probe_times_the_round_sequence(hip_library):
         sums.append(checksum)
     slot = cycles / (1 << 16)
     ghz = cycles / (ticks * 10.0)
-    assert 36 <= slot < 60, slot
+    assert 32 <= slot < 36, slot           # 36: the two-lane form's nine
     assert 0.8 < ghz < 2.6, ghz
     assert sums[0] != sums[1]
 
