@@ -202,16 +202,21 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
 // CUs full of them.  Pieces dealt to the XCDs in contiguous ranges ran at
 // 6.35 TB/s, so consecutive pieces go round robin.
 //
-// A gather's records are read next (by a scatter, the CRC32C or SHA-256
-// kernels, the copy engine), and the memory-side cache holds 256 MiB of what
-// was written last: up to kKeptBytes the records are written with ordinary
-// stores (kKeep), which leave them there, above that with nontemporal ones. A
-// scatter takes its blocks from the last to the first, so it meets the kept
-// ones first.  Gather then scatter: 604 MB in 16 KiB spans 434 -> 407 us, in 64
-// KiB spans 373 -> 360, 151 MB in 4 KiB spans 110 -> 93; the reversed order
-// alone gave nothing.  Alone, a gather of more than the cache holds is 5 %
-// slower with ordinary stores (604 MB 204 -> 215 us; 151 MB 52 -> 54), hence
-// the line at three times the cache, where a third of the records still hits.
+// A gather's records are written with ordinary stores up to kKeptBytes (kKeep):
+// the memory-side cache (256 MiB) takes what was written last and writes it out
+// later, while nontemporal stores go out at once.  Ordinary against nontemporal,
+// 16 KiB spans, packed buffers in rotation, us:
+//   * a gather and a scatter, the cache full of lines that were read: 604 MB 390
+//     against 414 (the gather 178 against 198, the scatter 212 and 215), 302 MB
+//     209 / 224, 151 MB 108 / 114, 37 MB 35 / 35; with a 0.5 GB read behind them
+//     487 / 510 (604 MB), so nothing was only put off;
+//   * the cache full of lines that another kernel wrote (a 1 GB fill), which the
+//     ordinary stores push out: 604 MB 421 / 416, 151 MB 119 / 115; with the
+//     read, which pushes them out otherwise, 518 / 561 and 238 / 261;
+//   * a gather and a CRC32C pass, after reads: 604 MB 312 / 299, 151 MB 90 / 92,
+//     1208 MB 633 / 586, where a scatter still gains (798 / 814).
+// The line, three times the cache: above it the CRC32C pass behind a hashed
+// save's gather loses more than a scatter gains.
 constexpr int kPieceBytes = 64 * 16;
 constexpr int64_t kKeptBytes = int64_t(768) << 20;
 
@@ -220,8 +225,7 @@ __device__ __forceinline__ void copy_piece(const int64_t* __restrict__ blocks, c
                                            const int64_t* __restrict__ bases, const int64_t* __restrict__ pitches,
                                            const int64_t* __restrict__ words, uint32_t pieces,
                                            char* __restrict__ records, int64_t record_pitch) {
-    const uint32_t b = kGather ? blockIdx.y : gridDim.y - 1 - blockIdx.y;
-    const uint32_t s = blockIdx.x / pieces, p = blockIdx.x - s * pieces;
+    const uint32_t b = blockIdx.y, s = blockIdx.x / pieces, p = blockIdx.x - s * pieces;
     const int64_t length = words[s] * 8, at = static_cast<int64_t>(p) * kPieceBytes;
     if (at >= length) return;
     const int64_t end = p + 1 == pieces || length - at < kPieceBytes ? length : at + kPieceBytes;

@@ -1,5 +1,5 @@
 """The gather's two stores (records kept in the memory-side cache, or streamed past it) at the line between them,
-and the scatter that reads them back from the last block on."""
+and the scatter that reads them back."""
 import pytest
 import torch
 
