@@ -2514,8 +2514,9 @@ uint32_t* static_crc_workspace() {
 // decode step whose workgroups are dealt evenly over the chip waits for the
 // ones on those CUs (the synthetic decode's median step went from 0.80 to
 // 0.75 ms beside hashed saves once the SHA-256 workgroups took whole CUs).
-// The cost is a few CUs (one per SHA-256 group of 64 records, one per copy
-// workgroup) that the engine's LDS-using kernels leave alone.
+// The cost is a few CUs (one per SHA-256 workgroup of 24 or 64 records, see
+// kShaQuadGroups, one per copy workgroup) that the engine's LDS-using kernels
+// leave alone.
 constexpr unsigned kCuLds = 160 * 1024;
 constexpr unsigned kCopyLdsFence = kCuLds;                                        // plain copies: no LDS of their own
 constexpr unsigned kCheckedLdsFence = kCuLds - sizeof(uint32_t) * kCheckedLdsWords;  // the checked copies' tables
@@ -2529,7 +2530,12 @@ static_assert(sizeof(ShaShape<ShaTwoLane>::Schedule) < kCuLds && sizeof(ShaShape
 // at once: every workgroup holds its CU for the whole launch, and the CUs are
 // the engine's too.  Both forms' times are one record's chain, whatever the
 // number of records, until a form runs out of CUs (records of 288 KiB: 4.50 ms
-// for 1536 in the quad form, 5.1 ms for 2000 in the two-lane form).
+// for 1536 in the quad form, 5.1 ms for 2000 in the two-lane form).  What the
+// CUs cost a decode beside them (reads of 5.6 TB/s, a median step of 0.649 ms
+// alone, range launches queued throughout): 512 records 0.655 ms on 22 quad CUs
+// and 0.652 on 8 two-lane ones, 1536 records 0.663 on 64 and 0.659 on 24 (p99
+// 0.674 and 0.665).  Past the line the quad form would take more than a quarter
+// of the chip for each session.
 constexpr int64_t kShaQuadGroups = 64;
 
 template <class Form>
