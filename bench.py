@@ -800,8 +800,9 @@ def disk_fork(args, caches):
 def run_rotating(args, hashed=None):
     """Qwen3-1.7B fp8-e4m3 sessions of 1k/2k/4k/8k tokens saved and restored round-robin from a side thread
     beside a synthetic 16-sequence decode on the compute stream (reference results/resume-phases.json:351,
-    396).  ``hashed`` (default: ``--digests``) has every save compute its CRC32C and SHA-256 on the GPU;
-    the last round's are then checked against the oracle's digests of the records."""
+    396).  ``hashed`` (default: ``--digests``) has every save compute its CRC32C and SHA-256, on the GPU
+    or, for few records, on host threads; the last round's are then checked against the oracle's digests of the
+    records."""
     import torch
     hashed = args.digests if hashed is None else hashed
     from kvsnap_amd import synth
@@ -1526,8 +1527,9 @@ def run_turns(args):
             "full_adopted_ms": median("full_ms"), "disk_delta_fenced_ms": median("disk_fenced_ms"),
             "disk_delta_written_ms": median("disk_ms"),
             "fence_speedup": round(median("full_fenced_ms") / median("delta_fenced_ms"), 2),
-            "note": "adopted = digests computed on the GPU and the blocks held by content id; a record's "
-                    "SHA-256 is one sequential chain, so both saves' adoption waits about one record's hash",
+            "note": "adopted = digests taken and the blocks held by content id; a full save's on the GPU, where a "
+                    "record's SHA-256 is one sequential chain, a turn's new blocks' on host threads "
+                    "(KVSNAP_HASH_THREADS)",
             "record_bytes": size, "start_tokens": start_tokens, "tokens_per_turn": turn_tokens, "turns": rows,
             "segments_equal": True, "layout": args.layout, "cpu_baseline": cpu}
 
