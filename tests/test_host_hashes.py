@@ -281,6 +281,9 @@ def test_the_rule(kernels, monkeypatch):
     assert threads(1) == threads(32) == 2 and threads(33) == 0
     monkeypatch.setattr(dataplane.os, "sched_getaffinity", lambda pid: {3})
     assert threads(16) == 1 and threads(17) == 0
+    monkeypatch.setattr(dataplane.os, "sched_getaffinity", lambda pid: set(range(512)))
+    monkeypatch.setattr(dataplane, "HASH_THREADS", 400)
+    assert threads(1) == 256
     monkeypatch.setattr(dataplane, "HASH_THREADS", 0)
     assert threads(1) == 0
     monkeypatch.setattr(dataplane, "HASH_THREADS", 2)
