@@ -288,7 +288,7 @@ def test_the_rule(kernels, monkeypatch):
     assert threads(1) == 0
     monkeypatch.setattr(dataplane, "HASH_THREADS", 2)
     plane.timer = object()
-    assert threads(1) == 1                  # a timer times what runs
+    assert threads(1) == 2                  # a timer times what runs
     plane.timer = None
     kernels.kvsnap_hash_records_available = lambda: 0
     assert threads(1) == 0
